@@ -124,7 +124,7 @@ typedef struct glx_td_params {
                           * Not supported by glx_batch_td_run. */
 } glx_td_params;
 
-/* nsteps TDGL steps in one persistent launch: per step up to max_sweeps psi
+/* nsteps TDGL steps in persistent launches: per step up to max_sweeps psi
  * sweeps and (if solveA) up to max_sweeps A sweeps, each sweep followed by a
  * grid barrier and the reference's stop rule, with no host round trip.
  * psi_bufs / ab_bufs are three same-sized buffers rotated in place of the
@@ -134,10 +134,15 @@ typedef struct glx_td_params {
  * 2*nsteps int32) receives (S_psi, S_A) per step.
  * Replaces the host loops TD.__iterate / __iterate_order_parameter_gpu /
  * __iterate_vector_potential_gpu, svirl/solvers/td.py:157-366, with the
- * A-source aliasing of td.py:264-303 kept. wg / wg_size select the
- * persistent grid of both solves (wg 0: the library default, two
- * workgroups per CU for the psi solve and three for the A solve, within
- * the co-resident limit). */
+ * A-source aliasing of td.py:264-303 kept. wg 0: the library's choice -
+ * grids that fit the registers of the chip (about 1.3 million nodes in
+ * FP32, 1.0 million in FP64) run all steps in one launch on register tiles,
+ * unless the run has Langevin noise, a fixed source, eqn 2 or profiling
+ * enabled; the others in one launch per solve on two workgroups per CU for
+ * psi and three for A (small grids: about 32 rows a wave). wg > 0: one
+ * launch per solve on that many workgroups of wg_size (256) threads. The
+ * fields and sweep counts are the same either way in FP64, within its
+ * rounding in FP32. */
 int glx_td_run(int prec, glx_grid g, const glx_td_params *p, const void *eps_map,
                const uint8_t *mt, void *const psi_bufs[3], int32_t *psi_cur,
                void *const ab_bufs[3], int32_t *ab_cur, void *rhs_psi, void *rhs_ab,
@@ -269,11 +274,13 @@ int glx_td_last_kernel_ms(float *ms);
  * reference; a measurement hook). While enabled, glx_td_run brackets every
  * psi-solve and A-solve launch with HIP events on the library stream;
  * glx_td_solve_ms returns the summed durations (ms) and launch counts of the
- * last glx_td_run call (zeros when profiling was off). */
+ * last glx_td_run call (zeros when profiling was off). A profiled run makes
+ * one launch per solve also where it would run on register tiles. */
 int glx_td_profile(int32_t enable);
 int glx_td_solve_ms(double *psi_ms, int32_t *psi_launches, double *a_ms, int32_t *a_launches);
 
-/* Memory passes of the last glx_td_run call (no counterpart in the
+/* Memory passes of the last glx_td_run call (a run on register tiles counts
+ * one per solve and redone solve; no counterpart in the
  * reference; a measurement hook, like glx_td_solve_ms): the psi solves'
  * passes over the fields (a fused pass of two or three sweeps counts once)
  * and the redone ones among them (a pass repeated up to an earlier sweep

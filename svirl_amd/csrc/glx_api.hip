@@ -136,15 +136,16 @@ int glx_init(int device) {
     g_ctx.env.passes = g_ctx.passes;
     g_ctx.env.grow = &g_ctx.grow;
     g_ctx.env.grow_bytes = &g_ctx.grow_bytes;
-    // library scratch layout: partials | result | arrive | rel | err | state | sweeps
+    // library scratch layout: partials | result | arrive | rel | chk | err | state | sweeps
     const size_t partials = sizeof(double) * 1024 * 32;
     const size_t result = sizeof(double) * 64;
     const size_t arrive = sizeof(unsigned long long) * MAX_GRID_BLOCKS;
     const size_t rel = sizeof(unsigned long long) * NREL * REL_STRIDE;
     const size_t err = 512;
+    const size_t chk = 4 * arrive;  // check and group words, two arrays of each
     const size_t state = 512;
     const size_t sweeps = sizeof(int) * 2 * SWEEPS_CAP;
-    const size_t total = partials + result + arrive + rel + err + state + sweeps;
+    const size_t total = partials + result + arrive + rel + chk + err + state + sweeps;
     if ((st = hipMalloc(&g_ctx.lib_scratch, total)) != hipSuccess) return check_hip(st, "hipMalloc(library scratch)");
     if ((st = hipMemset(g_ctx.lib_scratch, 0, total)) != hipSuccess) return check_hip(st, "hipMemset(library scratch)");
     char *p = (char *)g_ctx.lib_scratch;
@@ -154,6 +155,7 @@ int glx_init(int device) {
     e.result = (double *)p; p += result;
     e.arrive = (unsigned long long *)p; p += arrive;
     e.rel = (unsigned long long *)p; p += rel;
+    e.chk = (unsigned long long *)p; p += chk;
     e.err = (int *)p; p += err;
     e.state = (int *)p; p += state;
     e.sweeps = (int *)p; p += sweeps;

@@ -18,6 +18,7 @@ struct Env {
     unsigned long long *arrive; // grid barrier arrival words (MAX_GRID_BLOCKS)
     unsigned long long *rel;    // grid barrier release words (NREL, REL_STRIDE apart)
     int *err;                   // grid barrier error flag
+    unsigned long long *chk;    // check and group words of the tiled runs (4 * MAX_GRID_BLOCKS)
     int *state;              // persistent-kernel state
     int *sweeps;             // per-step sweep counts (capacity sweeps_cap steps)
     int sweeps_cap;

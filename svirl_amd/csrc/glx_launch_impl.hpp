@@ -2,14 +2,19 @@
 // glx_f32.hip.
 #pragma once
 
+#include <string.h>
+
 #include <algorithm>
+#include <limits>
 #include <mutex>
+#include <tuple>
 #include <unordered_map>
 #include <vector>
 
 #include "glx_fields.hpp"
 #include "glx_launch.hpp"
 #include "glx_td.hpp"
+#include "glx_tile.hpp"
 #include "glx_batch_cg.hpp"
 #include "glx_cg_rows.hpp"
 
@@ -160,14 +165,6 @@ int L<R>::a_sweep(const Env &e, glx_grid g, double dt, double kappa2, double rho
     return GLX_OK;
 }
 
-// The FP32-mixed run stores A as A - A_gauge(H) while it evolves A (exact
-// change of variable: the symmetric gauge is a fixed point of the A sweep
-// with psi = 0), so that the iterates stay small and float-resolved. FP64
-// runs, and FP32 runs that do not evolve A, keep the plain form (A is then
-// left bit-for-bit untouched).
-template <typename R> struct RunForm { static constexpr bool has_gauge = false; };
-template <> struct RunForm<float> { static constexpr bool has_gauge = true; };
-
 // Co-resident workgroups per CU of the psi solve kernel and of the A solve
 // kernels (the smaller of the plain and fixed-source forms).
 template <typename R, bool G> static int solve_occupancy2(int *psi_per_cu, int *a_per_cu) {
@@ -233,17 +230,17 @@ template <typename R> int L<R>::td_max_grid(const Env &e, int32_t wg_size, int32
     return GLX_OK;
 }
 
+// The arguments of a run's solve kernels, in the gauge-shifted form (G) or
+// the plain one.
 template <typename R, bool G>
-static int td_run_form(const Env &e, glx_grid g, const glx_td_params *p, const void *eps_map, const uint8_t *mt,
-                       void *const P[3], int32_t *pc, void *const Q[3], int32_t *qc, void *rhs_psi, void *rhs_ab,
-                       int32_t nsteps, int32_t *sweeps, int32_t wg, int32_t wg_a) {
-
+static TDSolveArgs<R> td_solve_args(const Env &e, const glx_grid &g, const glx_td_params *p, const void *eps_map,
+                                    const uint8_t *mt, void *const P[3], void *const Q[3], void *rhs_psi,
+                                    void *rhs_ab) {
     TDSolveArgs<R> T{};
     T.psi = make_psi_args<R>(g, p->dt, p->eps, eps_map, mt, nullptr, p->stop_psi, p->langevin_psi);
     T.A = make_a_args<R>(g, p->dt, p->kappa2, p->rho, p->H, mt, p->stop_A, p->langevin_A);
     const double Lx = g.dx * (g.Nx - 1), Ly = g.dy * (g.Ny - 1);
-    const double gH = G ? p->H : 0.0;
-    T.psi.gH = T.A.gH = gH;
+    T.psi.gH = T.A.gH = G ? p->H : 0.0;
     T.psi.gdx = T.A.gdx = g.dx;
     T.psi.gdy = T.A.gdy = g.dy;
     T.psi.gx0 = T.A.gx0 = 0.5 * Lx;
@@ -262,14 +259,62 @@ static int td_run_form(const Env &e, glx_grid g, const glx_td_params *p, const v
     T.sc.gs.err = e.err;
     T.sc.state = e.state;
     T.sc.sweeps = e.sweeps;
-    const long Nab = (long)(g.Nx - 1) * g.Ny + (long)g.Nx * (g.Ny - 1);
+    return T;
+}
 
+// A <-> A - A_g of the run's vector potential: buffer qc before the first
+// step (sign -1), the state's current one after the last (sign +1).
+template <typename R>
+static int td_gauge_shift(const Env &e, const glx_grid &g, const TDSolveArgs<R> &T, int qc, double sign) {
+    const long Nab = (long)(g.Nx - 1) * g.Ny + (long)g.Nx * (g.Ny - 1);
+    if (sign < 0.0)
+        hipLaunchKernelGGL(k_gauge_shift<R>, dim3(grid_blocks(Nab)), dim3(256), 0, e.stream, T.Q[qc], g.Nx, g.Ny,
+                           T.A.gH, g.dx, g.dy, T.A.gx0, T.A.gy0, sign);
+    else
+        hipLaunchKernelGGL(k_gauge_shift_state<R>, dim3(grid_blocks(Nab)), dim3(256), 0, e.stream, T.Q[0], T.Q[1],
+                           T.Q[2], e.state, g.Nx, g.Ny, T.A.gH, g.dx, g.dy, T.A.gx0, T.A.gy0, sign);
+    GLX_LAUNCH_CHECK("k_gauge_shift");
+    return GLX_OK;
+}
+
+// The end of a run: its state, error flag and sweep counts to the host.
+static int td_run_finish(const Env &e, int32_t nsteps, bool do_psi, bool do_A, int32_t *pc, int32_t *qc,
+                         int32_t *sweeps) {
+    int host_state[ST_WORDS] = {0};
+    int host_err = 0;
+    hipError_t st = hipMemcpyAsync(host_state, e.state, sizeof(int) * ST_WORDS, hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(&host_err, e.err, sizeof(int), hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(sweeps, e.sweeps, sizeof(int) * 2 * nsteps, hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
+    if (st != hipSuccess) return check_hip(st, "glx_td_run readback");
+    float kms = 0.f;
+    if (hipEventElapsedTime(&kms, e.kev0, e.kev1) == hipSuccess && e.last_kernel_ms) *e.last_kernel_ms = kms;
+    if (e.solve_ms && e.solve_n) {
+        e.solve_ms[0] = e.solve_ms[1] = 0.0;
+        e.solve_n[0] = e.solve_n[1] = 0;
+    }
+    if (host_err) return set_error(GLX_E_TIMEOUT, "glx_td_run: grid barrier timed out in step %d of %d", host_state[ST_ERRSTEP], nsteps);
+    if (!do_psi)
+        for (int k = 0; k < nsteps; ++k) sweeps[2 * k] = 0;
+    if (!do_A)
+        for (int k = 0; k < nsteps; ++k) sweeps[2 * k + 1] = 0;
+    *pc = host_state[ST_PSI];
+    *qc = host_state[ST_AB];
+    if (e.passes)
+        for (int k = 0; k < 5; ++k) e.passes[k] = host_state[ST_PASS_PSI + k];
+    return GLX_OK;
+}
+
+template <typename R, bool G>
+static int td_run_form(const Env &e, glx_grid g, const glx_td_params *p, const void *eps_map, const uint8_t *mt,
+                       void *const P[3], int32_t *pc, void *const Q[3], int32_t *qc, void *rhs_psi, void *rhs_ab,
+                       int32_t nsteps, int32_t *sweeps, int32_t wg, int32_t wg_a) {
+    TDSolveArgs<R> T = td_solve_args<R, G>(e, g, p, eps_map, mt, P, Q, rhs_psi, rhs_ab);
     hipLaunchKernelGGL(k_td_reset, dim3(1), dim3(256), 0, e.stream, T.sc, (int)*pc, (int)*qc, e.abort_next ? 1 : 0);
     GLX_LAUNCH_CHECK("k_td_reset");
     if (G) {
-        hipLaunchKernelGGL(k_gauge_shift<R>, dim3(grid_blocks(Nab)), dim3(256), 0, e.stream, T.Q[*qc], g.Nx, g.Ny, gH,
-                           g.dx, g.dy, 0.5 * Lx, 0.5 * Ly, -1.0);
-        GLX_LAUNCH_CHECK("k_gauge_shift");
+        int rc = td_gauge_shift<R>(e, g, T, *qc, -1.0);
+        if (rc) return rc;
     }
     hipError_t est = hipEventRecord(e.kev0, e.stream);
     if (est != hipSuccess) return check_hip(est, "hipEventRecord");
@@ -304,48 +349,172 @@ static int td_run_form(const Env &e, glx_grid g, const glx_td_params *p, const v
     est = hipEventRecord(e.kev1, e.stream);
     if (est != hipSuccess) return check_hip(est, "hipEventRecord");
     if (G) {
-        hipLaunchKernelGGL(k_gauge_shift_state<R>, dim3(grid_blocks(Nab)), dim3(256), 0, e.stream, T.Q[0], T.Q[1], T.Q[2],
-                           e.state, g.Nx, g.Ny, gH, g.dx, g.dy, 0.5 * Lx, 0.5 * Ly, 1.0);
-        GLX_LAUNCH_CHECK("k_gauge_shift_state");
+        int rc = td_gauge_shift<R>(e, g, T, 0, 1.0);
+        if (rc) return rc;
     }
-    int host_state[ST_WORDS] = {0};
-    int host_err = 0;
-    hipError_t st = hipMemcpyAsync(host_state, e.state, sizeof(int) * ST_WORDS, hipMemcpyDeviceToHost, e.stream);
-    if (st == hipSuccess) st = hipMemcpyAsync(&host_err, e.err, sizeof(int), hipMemcpyDeviceToHost, e.stream);
-    if (st == hipSuccess) st = hipMemcpyAsync(sweeps, e.sweeps, sizeof(int) * 2 * nsteps, hipMemcpyDeviceToHost, e.stream);
-    if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
-    if (st != hipSuccess) return check_hip(st, "glx_td_run readback");
-    float kms = 0.f;
-    if (hipEventElapsedTime(&kms, e.kev0, e.kev1) == hipSuccess && e.last_kernel_ms) *e.last_kernel_ms = kms;
-    if (e.solve_ms && e.solve_n) {
-        e.solve_ms[0] = e.solve_ms[1] = 0.0;
-        e.solve_n[0] = e.solve_n[1] = 0;
-        if (prof) {
-            int k = 0;
-            for (int step = 0; step < nsteps; ++step)
-                for (int kind = 0; kind < 2; ++kind) {
-                    if ((kind == 0 && !do_psi) || (kind == 1 && !do_A)) continue;
-                    float ms = 0.f;
-                    if (hipEventElapsedTime(&ms, e.tev[k], e.tev[k + 1]) == hipSuccess) {
-                        e.solve_ms[kind] += ms;
-                        e.solve_n[kind] += 1;
-                    }
-                    k += 2;
+    const int rc = td_run_finish(e, nsteps, do_psi, do_A, pc, qc, sweeps);
+    if (prof && e.solve_ms && e.solve_n) {
+        int k = 0;
+        for (int step = 0; step < nsteps; ++step)
+            for (int kind = 0; kind < 2; ++kind) {
+                if ((kind == 0 && !do_psi) || (kind == 1 && !do_A)) continue;
+                float ms = 0.f;
+                if (hipEventElapsedTime(&ms, e.tev[k], e.tev[k + 1]) == hipSuccess) {
+                    e.solve_ms[kind] += ms;
+                    e.solve_n[kind] += 1;
                 }
-        }
+                k += 2;
+            }
     }
-    if (host_err) return set_error(GLX_E_TIMEOUT, "glx_td_run: grid barrier timed out in step %d of %d", host_state[ST_ERRSTEP], nsteps);
-    if (!do_psi)
-        for (int k = 0; k < nsteps; ++k) sweeps[2 * k] = 0;
-    if (!do_A)
-        for (int k = 0; k < nsteps; ++k) sweeps[2 * k + 1] = 0;
-    *pc = host_state[ST_PSI];
-    *qc = host_state[ST_AB];
-    if (e.passes)
-        for (int k = 0; k < 5; ++k) e.passes[k] = host_state[ST_PASS_PSI + k];
+    return rc;
+}
+
+// ---- runs on register tiles ------------------------------------------------------
+
+// The smallest change that counts as not converged: scaled_residual(r) >=
+// 10000 from there on (it is non-decreasing in r), found by bisection over
+// the bit patterns of the non-negative numbers.
+template <typename R> static R stop_threshold(double stop_eps) {
+    using U = std::conditional_t<sizeof(R) == 8, uint64_t, uint32_t>;
+    auto open = [&](R r) {
+        R v = R(1.0e4 * double(r) / stop_eps);
+        if (v > R(1.0e8)) v = R(1.0e8);
+        return int(v) >= 10000;
+    };
+    auto of = [](U u) { R r; memcpy(&r, &u, sizeof r); return r; };
+    U lo = 0, hi;
+    const R inf = std::numeric_limits<R>::infinity();
+    memcpy(&hi, &inf, sizeof hi);
+    while (hi - lo > 1) {
+        const U mid = lo + (hi - lo) / 2;
+        if (open(of(mid))) hi = mid;
+        else lo = mid;
+    }
+    return of(hi);
+}
+
+// The words the tiles of a launch meet through: check words, then group words.
+static TileSync tile_sync(const Env &e) {
+    unsigned long long *c = e.chk, *g = e.chk + 2 * MAX_GRID_BLOCKS;
+    return {e.arrive, {c, c + MAX_GRID_BLOCKS}, {g, g + MAX_GRID_BLOCKS}, e.err};
+}
+
+// Zero the words the first nwg tiles of a run meet through and set the
+// run's state (k_td_reset's part for the row-marching solves).
+static __global__ void k_tile_reset(TileSync ts, int nwg, int *state, int pc, int qc, int err0) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nwg) ts.flag[k] = ts.chk[0][k] = ts.chk[1][k] = 0ull;
+    if (k * TILE_GROUP < nwg) ts.grp[0][k] = ts.grp[1][k] = 0ull;
+    if (k < ST_WORDS) state[k] = k == ST_PSI ? pc : (k == ST_AB ? qc : 0);
+    if (k == 0) *ts.err = err0;
+}
+
+// The tiles of a shape that cover a grid, and whether that many workgroups
+// are co-resident.
+struct TilePlan {
+    int ntx, nty;
+    bool fits;
+};
+template <typename R, bool WITHA, typename SH> static int tile_plan(const Env &e, const glx_grid &g, TilePlan *pl) {
+    static int per_cu = 0;  // queried once
+    if (per_cu <= 0) {
+        int m = 0;
+        hipError_t st = hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, k_td_tiles<R, WITHA, SH>, SH::NW * WAVE, 0);
+        if (st != hipSuccess) return check_hip(st, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+        per_cu = m;
+    }
+    pl->ntx = (g.Nx + SH::COLS - 1) / SH::COLS;
+    pl->nty = (g.Ny + SH::ROWS - 1) / SH::ROWS;
+    pl->fits = (long)pl->ntx * pl->nty <= std::min((long)per_cu * e.num_cus, (long)MAX_GRID_BLOCKS);
     return GLX_OK;
 }
 
+// f(integral_constant k) for every k of a shape list.
+template <typename Shapes, typename F, size_t... K> static void each_shape_of(F &&f, std::index_sequence<K...>) {
+    (f(std::integral_constant<size_t, K>{}), ...);
+}
+template <typename Shapes, typename F> static void each_shape(F &&f) {
+    each_shape_of<Shapes>(f, std::make_index_sequence<std::tuple_size_v<Shapes>>{});
+}
+
+// What a sweep costs on a shape, in rows of one wave per SIMD: the rows of
+// the workgroups that share a CU, what a sweep costs beside its rows, and
+// its share of an exchange of rings (fitted to the times of every shape on
+// grids of 33^2 to 1025^2; the choice is within 7% of the fastest shape
+// there but for FP64 at 385^2, 13%).
+template <typename SH> static double tile_cost(const Env &e, const TilePlan &pl) {
+    const double per_cu = double((pl.ntx * pl.nty + e.num_cus - 1) / e.num_cus);
+    return per_cu * SH::NR * (SH::NW / 4) + 4.0 + 60.0 / SH::H;
+}
+
+template <typename R, bool WITHA, typename SH>
+static int td_run_tiles(const Env &e, const TilePlan &pl, glx_grid g, const glx_td_params *p, const void *eps_map,
+                        const uint8_t *mt, void *const P[3], int32_t *pc, void *const Q[3], int32_t *qc,
+                        int32_t nsteps, int32_t *sweeps) {
+    constexpr bool G = WITHA && RunForm<R>::has_gauge;
+    const int nwg = pl.ntx * pl.nty;
+    TDSolveArgs<R> T = td_solve_args<R, G>(e, g, p, eps_map, mt, P, Q, nullptr, nullptr);
+    const TileSync ts = tile_sync(e);
+    hipLaunchKernelGGL(k_tile_reset, dim3((nwg + 255) / 256), dim3(256), 0, e.stream, ts, nwg, e.state, (int)*pc,
+                       (int)*qc, e.abort_next ? 1 : 0);
+    GLX_LAUNCH_CHECK("k_tile_reset");
+    int rc = G ? td_gauge_shift<R>(e, g, T, *qc, -1.0) : GLX_OK;
+    if (rc) return rc;
+    hipError_t st = hipEventRecord(e.kev0, e.stream);
+    if (st != hipSuccess) return check_hip(st, "hipEventRecord");
+    hipLaunchKernelGGL((k_td_tiles<R, WITHA, SH>), dim3(nwg), dim3(SH::NW * WAVE), 0, e.stream, T, ts, pl.ntx,
+                       pl.nty, (int)nsteps, stop_threshold<R>(T.psi.stop_eps), stop_threshold<R>(T.A.stop_eps));
+    GLX_LAUNCH_CHECK("k_td_tiles");
+    st = hipEventRecord(e.kev1, e.stream);
+    if (st != hipSuccess) return check_hip(st, "hipEventRecord");
+    rc = G ? td_gauge_shift<R>(e, g, T, 0, 1.0) : GLX_OK;
+    if (rc) return rc;
+    return td_run_finish(e, nsteps, true, WITHA, pc, qc, sweeps);
+}
+
+// The tile shapes (rows per wave, halo, waves) of a precision. Few rows and
+// a narrow halo where the grid is small: more workgroups, each sweep short.
+// Many rows and waves where it is large: less of a tile is halo, and more
+// grids fit. The registers end the list: FP32 takes nine a node and spills
+// from 18 rows on, FP64 fourteen (and 24 bytes of LDS), from 9 on in the psi
+// sweeps. Measured per step (about 22 psi and 4 A sweeps; kappa = 5), row-marching
+// solves against tiles: FP32 129^2 276 / 39 us, 513^2 305 / 69, 1025^2 319 /
+// 113; FP64 129^2 444 / 51, 513^2 470 / 95, 771 x 1283 506 / 241.
+template <typename R> struct TileShapes { using list = std::tuple<TileOf<4, 4, 4>, TileOf<8, 6, 4>, TileOf<14, 8, 8>, TileOf<16, 8, 8>>; };
+template <> struct TileShapes<double> { using list = std::tuple<TileOf<4, 4, 4>, TileOf<5, 5, 8>, TileOf<8, 6, 8>, TileOf<10, 4, 8>>; };
+
+// Run on register tiles if the grid fits some shape: *done tells whether it
+// did.
+template <typename R, bool WITHA>
+static int td_try_tiles(const Env &e, glx_grid g, const glx_td_params *p, const void *eps_map, const uint8_t *mt,
+                        void *const P[3], int32_t *pc, void *const Q[3], int32_t *qc, int32_t nsteps, int32_t *sweeps,
+                        bool *done) {
+    using Shapes = typename TileShapes<R>::list;
+    int rc = GLX_OK;
+    double best = 0.0;
+    int pick = -1;
+    TilePlan plan{};
+    each_shape<Shapes>([&](auto k) {
+        using T = std::tuple_element_t<k, Shapes>;
+        TilePlan pl{};
+        if (!rc) rc = tile_plan<R, WITHA, T>(e, g, &pl);
+        if (rc || !pl.fits) return;
+        const double cost = tile_cost<T>(e, pl);
+        if (pick < 0 || cost < best) {
+            best = cost;
+            pick = (int)k;
+            plan = pl;
+        }
+    });
+    if (rc || pick < 0) return rc;
+    *done = true;
+    each_shape<Shapes>([&](auto k) {
+        using T = std::tuple_element_t<k, Shapes>;
+        if ((int)k == pick)
+            rc = td_run_tiles<R, WITHA, T>(e, plan, g, p, eps_map, mt, P, pc, Q, qc, nsteps, sweeps);
+    });
+    return rc;
+}
 
 template <typename R>
 int L<R>::td_run(const Env &e, glx_grid g, const glx_td_params *p, const void *eps_map, const uint8_t *mt,
@@ -366,17 +535,32 @@ int L<R>::td_run(const Env &e, glx_grid g, const glx_td_params *p, const void *e
     int32_t maxg = 0;
     int rc = td_max_grid(e, wg_size, &maxg);
     if (rc) return rc;
-    // Default grids, the measured optima at 4097^2: two workgroups per CU
-    // for the psi solve, three for the A solve, each within its own kernel's
-    // co-resident limit (maxg, the smaller of the two, bounds an explicit wg,
-    // which applies to both).
+    // Default: register tiles where the grid fits them and the run has none
+    // of what they leave out; else the row-marching solves, about 32 rows per
+    // wave for small grids and from there the measured optima at 4097^2: two
+    // workgroups per CU for the psi solve, three for the A solve, each within
+    // its own kernel's co-resident limit (maxg, the smaller of the two, bounds
+    // an explicit wg, which applies to both).
+    const bool noise = p->langevin_psi > 1.0e-32 || (p->solveA && p->langevin_A > 1.0e-32);
+    if (wg <= 0 && p->eqn != 2 && !noise && !p->a_src && !e.td_profile) {
+        bool done = false;
+        rc = (p->solveA && p->eqn == 0)
+                 ? td_try_tiles<R, true>(e, g, p, eps_map, mt, P, pc, Q, qc, nsteps, sweeps, &done)
+                 : td_try_tiles<R, false>(e, g, p, eps_map, mt, P, pc, Q, qc, nsteps, sweeps, &done);
+        if (rc || done) return rc;
+    }
     int32_t wg_a = wg;
     if (wg <= 0) {
         int32_t psi_max = 0, a_max = 0;
         rc = solve_grids<R>(e, &psi_max, &a_max);
         if (rc) return rc;
-        wg = std::min(psi_max, 2 * e.num_cus);
-        wg_a = std::min(a_max, 3 * e.num_cus);
+        const long waves = std::max(1L, (long)nstrips_of<1>(g.Nx) * g.Ny / 32);
+        wg = (int)std::max(1L, std::min((long)maxg, (waves + 3) / 4));
+        wg_a = wg;
+        if (wg >= std::min(maxg, 2 * e.num_cus)) {
+            wg = std::min(psi_max, 2 * e.num_cus);
+            wg_a = std::min(a_max, 3 * e.num_cus);
+        }
     }
     if (wg > maxg) return set_error(GLX_E_ARG, "glx_td_run: grid %d exceeds co-resident limit %d", wg, maxg);
     const bool evolves_A = p->solveA && p->eqn != 1;

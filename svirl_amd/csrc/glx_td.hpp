@@ -60,6 +60,14 @@ template <typename R> struct ASweepArgs {
     double gH, gdx, gdy, gx0, gy0;  // as in PsiSweepArgs
 };
 
+// The FP32-mixed run stores A as A - A_gauge(H) while it evolves A (exact
+// change of variable: the symmetric gauge is a fixed point of the A sweep
+// with psi = 0), so that the iterates stay small and float-resolved. FP64
+// runs, and FP32 runs that do not evolve A, keep the plain form (A is then
+// left bit-for-bit untouched).
+template <typename R> struct RunForm { static constexpr bool has_gauge = false; };
+template <> struct RunForm<float> { static constexpr bool has_gauge = true; };
+
 // Symmetric gauge of field H (the one svirl builds, params.py:159-167) on
 // link a(c, j) and b(c, j): a_g = -H/2 (y_j - Ly/2), b_g = H/2 (x_c - Lx/2).
 __device__ __forceinline__ double gauge_a(double H, double dy, double y0, int j) { return -0.5 * H * (double(j) * dy - y0); }

@@ -45,7 +45,7 @@ class TD:
         self._rhs_psi = None
         self._rhs_ab = None
         self.sweeps = []          # (S_psi, S_A) per time step
-        self.wg = 0               # persistent grid (0: chosen per grid size)
+        self.wg = 0               # row-marching solves on so many workgroups (0: the library's choice)
         self.steps_per_launch = None
         self.td_energies = []
 
@@ -172,7 +172,6 @@ class TD:
         Pp = (ctypes.c_void_p * 3)(*[b.ptr for b in P])
         Qp = (ctypes.c_void_p * 3)(*[b.ptr for b in Q])
         cpc, cqc = ctypes.c_int32(pc), ctypes.c_int32(qc)
-        wg = self.wg or self._default_wg()
         chunk = self._launch_steps()
         done = 0
         while done < nsteps:
@@ -181,7 +180,7 @@ class TD:
             sw = (ctypes.c_int32 * (2 * n))()
             nat.call("glx_td_run", self.par.prec, g, ctypes.byref(prm), nat.ptr(p.linear_coefficient_h()),
                      nat.ptr(self.mesh.material_tiling_h()), Pp, ctypes.byref(cpc), Qp, ctypes.byref(cqc),
-                     nat.ptr(self._rhs_psi), nat.ptr(self._rhs_ab), n, sw, wg, 256)
+                     nat.ptr(self._rhs_psi), nat.ptr(self._rhs_ab), n, sw, self.wg, 256)
             self._finish(P, cpc.value, Q, cqc.value, np.frombuffer(sw, dtype=np.int32), eqn_code)
             done += n
 
