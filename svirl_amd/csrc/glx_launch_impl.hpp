@@ -478,9 +478,9 @@ static int td_run_tiles(const Env &e, const TilePlan &pl, glx_grid g, const glx_
 // grids fit. The registers end the list: FP32 takes nine a node and spills
 // from 18 rows on, FP64 fourteen (and 24 bytes of LDS), from 9 on in the psi
 // sweeps. Measured per step (about 22 psi and 4 A sweeps; kappa = 5), row-marching
-// solves against tiles: FP32 129^2 276 / 39 us, 513^2 305 / 69, 1025^2 319 /
-// 113; FP64 129^2 444 / 51, 513^2 470 / 95, 771 x 1283 506 / 241.
-template <typename R> struct TileShapes { using list = std::tuple<TileOf<4, 4, 4>, TileOf<8, 6, 4>, TileOf<14, 8, 8>, TileOf<16, 8, 8>>; };
+// solves against tiles: FP32 129^2 276 / 43 us, 513^2 305 / 57, 1025^2 319 /
+// 94; FP64 129^2 444 / 48, 513^2 470 / 80, 771 x 1283 506 / 174.
+template <typename R> struct TileShapes { using list = std::tuple<TileOf<4, 4, 4>, TileOf<8, 6, 4>, TileOf<12, 8, 4>, TileOf<14, 8, 8>, TileOf<16, 8, 8>>; };
 template <> struct TileShapes<double> { using list = std::tuple<TileOf<4, 4, 4>, TileOf<5, 5, 8>, TileOf<8, 6, 8>, TileOf<10, 4, 8>>; };
 
 // Run on register tiles if the grid fits some shape: *done tells whether it

@@ -13,12 +13,20 @@
 // go on. Link factors, right-hand sides and diagonals stay in registers for
 // the whole solve, and one launch runs all steps of a run.
 //
-// The arithmetic is that of the row-marching passes (psi_rows, a_rows):
-// FP64 results and every sweep count equal theirs to the bit. The quotient
+// The FP64 arithmetic is that of the row-marching passes (psi_rows, a_rows):
+// results and every sweep count equal theirs to the bit. The quotient
 // n / den is formed from the rounded reciprocal r of den (once per step):
 // q = n r, then q + r (n - q den) with one fma each, which is the IEEE
 // quotient but for cases a 2^-52 part of inputs can reach (v_div_fixup
 // covers zeros, infinities and NaN), in 4 instructions against about 12.
+//
+// FP32 psi solves carry the change d of a sweep and the sum D of the changes
+// instead of psi and its right-hand side: the solve is linear in psi, so
+// d' = M d, and psi^{n+1} = psi^n + D. That costs the same registers and
+// instructions, D is rounded at the size of a step's change (a hundredth of
+// psi's), and the stop rule's 1e-6 is tested on values whose own rounding is
+// 1e-13, where the difference of two rounded iterates is off by up to 1e-7
+// and makes about 2 of 100 solves go a sweep too far.
 #pragma once
 
 #include "glx_td.hpp"
@@ -29,6 +37,7 @@ namespace glx {
 template <int NR_, int H_, int NW_> struct TileOf {
     static constexpr int NR = NR_, H = H_, NW = NW_;
     static constexpr int COLS = WAVE - 2 * H, ROWS = NW * NR - 2 * H;  // of the tile's own
+    static_assert(NW >= 4 && H <= NR && ROWS > 0, "tile shape");
 };
 
 // What the tiles of one instance need to meet: a flag word per workgroup
@@ -48,8 +57,10 @@ struct TileTeam {
 
 template <typename R, typename SH> struct TileLds {
     static constexpr int NR = SH::NR, NW = SH::NW;
-    // first and last rows of every wave, two copies used in turn
-    cplx<R> edge[2][NW][2][WAVE];
+    // first and last rows of every wave (slots 2 w + 1 and 2 w + 2) between
+    // two rows of zeros that stand for what lies beyond the tile, two copies
+    // used in turn
+    cplx<R> edge[2][2 * NW + 2][WAVE];
     // FP64: the right-hand side and the diagonal of every node (each lane
     // reads its own)
     static constexpr int KW = std::is_same<R, double>::value ? NW : 1;
@@ -120,6 +131,15 @@ template <typename T> __device__ __forceinline__ T fresh_args(const T *p) {
     for (unsigned k = 0; k < sizeof(T) / 4; ++k) d[k] = w[k];
     return v;
 }
+
+// One argument field through the scalar cache. What the tiles branch on
+// and index with (these, buffer indices, the words of a meeting) is made
+// uniform explicitly: read from memory or LDS like lane data it would turn
+// every loop of a solve into one over execution masks.
+template <typename T> __device__ __forceinline__ T arg(const T *p) {
+    return *(const __attribute__((address_space(4))) T *)(uintptr_t)p;
+}
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // x where bit r of `on` is set, else 0.
 __device__ __forceinline__ float tile_mask(float x, unsigned on, int r) {
@@ -209,7 +229,9 @@ __device__ __forceinline__ double tile_div(double n, double den, double r) {
 // The lane's part of a psi solve: psi, the link factors of a(c, j) and
 // b(c, j) (FP32: scaled by dt/dx^2, dt/dy^2; zero where the link touches no
 // material), those of b above row 0, and the diagonals. FP32 keeps
-// 1/den and rhs/den (psi_apply_folded), FP64 1/den and, in LDS, rhs and den.
+// 1/den, and the change of the last sweep in p (psi^n before the first) and
+// the sum of all in rd (rhs/den - psi^n before the first); FP64 1/den and, in
+// LDS, rhs and den.
 template <typename R, typename SH> struct PsiTile {
     static constexpr int NR = SH::NR;
     cplx<R> p[NR], rd[NR];
@@ -323,7 +345,7 @@ __device__ __forceinline__ void tile_psi_load(const PsiSweepArgs<R> *Ap, const c
         const cplx<R> rh = {inside ? t.p[r].re : R(0), inside ? t.p[r].im : R(0)};
         if constexpr (FOLD) {
             t.rden[r] = den;
-            t.rd[r] = {rh.re * den, rh.im * den};
+            t.rd[r] = {fmaf(rh.re, den, -t.p[r].re), fmaf(rh.im, den, -t.p[r].im)};
         } else {
             t.rden[r] = R(1) / den;
             S.rhs[X.w][r][X.lane] = rh;
@@ -335,8 +357,9 @@ __device__ __forceinline__ void tile_psi_load(const PsiSweepArgs<R> *Ap, const c
     }
 }
 
-// One node: psi^{j+1} from its own value, the rows below and above it (pm,
-// pp) and the lanes either side; (cm, sm) are the factors of the link below.
+// One node: psi^{j+1} (FP32: its neighbours' part in it) from its own value,
+// the rows below and above it (pm, pp) and the lanes either side; (cm, sm)
+// are the factors of the link below.
 template <typename R, typename SH>
 __device__ __forceinline__ cplx<R> tile_psi_node(const PsiSweepArgs<R> &A, const PsiTile<R, SH> &t, int r,
                                                  const cplx<R> &p, const cplx<R> &pm, const cplx<R> &pp, R cm, R sm,
@@ -359,7 +382,7 @@ __device__ __forceinline__ cplx<R> tile_psi_node(const PsiSweepArgs<R> &A, const
         im = fmaf(cb, pp.im, im);
         re = fmaf(sb, pp.im, re);
         im = fmaf(-sb, pp.re, im);
-        return {fmaf(re, t.rden[r], t.rd[r].re), fmaf(im, t.rden[r], t.rd[r].im)};
+        return {re, im};
     } else {
         const R m0r = shfl_up1(l_re), m0i = shfl_up1(l_im);
         const R p0r = ca * pr_re + sa * pr_im, p0i = ca * pr_im - sa * pr_re;
@@ -396,43 +419,62 @@ template <typename R> struct TileRes {
 template <typename R, typename SH>
 __device__ __forceinline__ void tile_edges_out(TileLds<R, SH> &S, int par, const TileCtx &X, const cplx<R> &lo,
                                                const cplx<R> &hi) {
-    S.edge[par][X.w][0][X.lane] = lo;
-    S.edge[par][X.w][1][X.lane] = hi;
+    S.edge[par][2 * X.w + 1][X.lane] = lo;
+    S.edge[par][2 * X.w + 2][X.lane] = hi;
 }
 
-// n psi sweeps on the tile; bit s of the result: sweep s left a change of at
+// n psi sweeps on the tile, the first of them the solve's first one or not
+// (FP32); bit s of the result: sweep s left a change of at
 // least thr at some node of the tile that belongs to this wave. `par` is the
 // LDS copy the first sweep reads (the caller's edges are there, behind a
 // barrier) and, on return, the one to be used next.
 template <typename R, typename SH>
 __device__ __forceinline__ unsigned tile_psi_sweeps(const PsiSweepArgs<R> *Ap, PsiTile<R, SH> &t, TileLds<R, SH> &S,
-                                                    const TileCtx &X, int n, R thr, int &par) {
+                                                    const TileCtx &X, int n, R thr, int &par_, bool first) {
     constexpr int NR = SH::NR;
+    int par = uniform(par_);
     constexpr bool F64 = std::is_same<R, double>::value;
     const PsiSweepArgs<R> A = fresh_args(Ap);
     unsigned bits = 0u;
-    const cplx<R> zero = {R(0), R(0)};
     const cplx<R>(*rl)[WAVE] = S.rhs[F64 ? X.w : 0];
     const R(*dl)[WAVE] = S.den[F64 ? X.w : 0];
     for (int s = 0; s < n; ++s) {
         // the rows above and below the wave's (unknown beyond the tile)
-        cplx<R> up = zero, dn = zero;
-        if (!X.first()) up = S.edge[par][X.w - 1][1][X.lane];
-        if (!X.last<SH>()) dn = S.edge[par][X.w + 1][0][X.lane];
+        const cplx<R> up = S.edge[par][2 * X.w][X.lane], dn = S.edge[par][2 * X.w + 3][X.lane];
         TileRes<R> res{R(0), R(0), R(0), R(0)};
         auto node = [&](int r, const cplx<R> &p, const cplx<R> &pm, const cplx<R> &pp, R cm, R sm) {
             const cplx<R> q = tile_psi_node<R, SH>(A, t, r, p, pm, pp, cm, sm, rl[F64 ? r : 0][X.lane],
                                                  dl[F64 ? r : 0][X.lane]);
-            res.template add<SH>(r, fmax(fabs(q.re - p.re), fabs(q.im - p.im)));
-            return q;
+            if constexpr (F64) {
+                res.template add<SH>(r, fmax(fabs(q.re - p.re), fabs(q.im - p.im)));
+                return q;
+            } else {
+                t.rd[r] = {fmaf(q.re, t.rden[r], t.rd[r].re), fmaf(q.im, t.rden[r], t.rd[r].im)};
+                const cplx<R> d = {q.re * t.rden[r], q.im * t.rden[r]};
+                res.template add<SH>(r, fmax(fabs(d.re), fabs(d.im)));
+                return d;
+            }
         };
-        cplx<R> prev = up;
+        // rows 1 .. NR-1, then row 0: `up` and `dn` have the middle rows to
+        // arrive in
+        const cplx<R> old0 = t.p[0], old1 = t.p[1];
+        cplx<R> prev = old0;
 #pragma unroll
-        for (int r = 0; r < NR; ++r) {
+        for (int r = 1; r < NR; ++r) {
             const cplx<R> cur = t.p[r];
-            t.p[r] = node(r, cur, prev, r + 1 < NR ? t.p[r + 1 < NR ? r + 1 : r] : dn, r > 0 ? t.cb[r > 0 ? r - 1 : 0] : t.cbu,
-                          r > 0 ? t.sb[r > 0 ? r - 1 : 0] : t.sbu);
+            t.p[r] = node(r, cur, prev, r + 1 < NR ? t.p[r + 1 < NR ? r + 1 : r] : dn, t.cb[r - 1], t.sb[r - 1]);
             prev = cur;
+        }
+        t.p[0] = node(0, old0, up, old1, t.cbu, t.sbu);
+        if constexpr (!F64) {
+            if (first && s == 0) {  // the first change has the own value's part too
+                res = {R(0), R(0), R(0), R(0)};
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    t.p[r] = t.rd[r];
+                    res.template add<SH>(r, fmax(fabs(t.p[r].re), fabs(t.p[r].im)));
+                }
+            }
         }
         par ^= 1;
         tile_edges_out<R, SH>(S, par, X, t.p[0], t.p[NR - 1]);
@@ -440,6 +482,7 @@ __device__ __forceinline__ unsigned tile_psi_sweeps(const PsiSweepArgs<R> *Ap, P
         bits |= __ballot(open) != 0ull ? 1u << s : 0u;
         __syncthreads();
     }
+    par_ = par;
     return bits;
 }
 
@@ -587,22 +630,25 @@ __device__ __forceinline__ void tile_a_sweep(const ASweepArgs<R> &A, ATile<R, SH
         }
         res.template add<SH>(r, fmax(fabs(va - a), fabs(vb - b)));
     };
-    R pa = up.re, pb = up.im;
+    const R a0 = t.a[0], b0 = t.b[0], a1 = t.a[1];
+    R pa = a0, pb = b0;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
+    for (int r = 1; r < NR; ++r) {
         const R a = t.a[r], b = t.b[r];
         links(r, a, b, pa, pb, r + 1 < NR ? t.a[r + 1 < NR ? r + 1 : r] : dn.re, t.a[r], t.b[r]);
         pa = a;
         pb = b;
     }
+    links(0, a0, b0, up.re, up.im, a1, t.a[0], t.b[0]);
 }
 
 // n A sweeps; result as tile_psi_sweeps. The LDS edges hold (a, b) of a
 // wave's first and last rows.
 template <typename R, typename SH>
 __device__ __forceinline__ unsigned tile_a_sweeps(const ASweepArgs<R> *Ap, ATile<R, SH> &t, TileLds<R, SH> &S,
-                                                  const TileCtx &X, int n, R thr, int &par, R rden_a, R rden_b) {
+                                                  const TileCtx &X, int n, R thr, int &par_, R rden_a, R rden_b) {
     constexpr int NR = SH::NR;
+    int par = uniform(par_);
     const ASweepArgs<R> A = fresh_args(Ap);
     unsigned bits = 0u;
     // dt rho kappa^2 times the ghost factor of the b links' column; 0 where
@@ -610,11 +656,8 @@ __device__ __forceinline__ unsigned tile_a_sweeps(const ASweepArgs<R> *Ap, ATile
     const R Ka = X.hasa(A.Nx) ? A.dt_rho_kappa2 : R(0);
     const R Kb = X.col(A.Nx) ? ((X.c == 0 || X.c + 1 == A.Nx) ? R(2) * A.dt_rho_kappa2 : A.dt_rho_kappa2) : R(0);
     const bool edge = X.j0 < 1 || X.j0 + NR > A.Ny - 1;
-    const cplx<R> zero = {R(0), R(0)};
     for (int s = 0; s < n; ++s) {
-        cplx<R> up = zero, dn = zero;
-        if (!X.first()) up = S.edge[par][X.w - 1][1][X.lane];
-        if (!X.last<SH>()) dn = S.edge[par][X.w + 1][0][X.lane];
+        const cplx<R> up = S.edge[par][2 * X.w][X.lane], dn = S.edge[par][2 * X.w + 3][X.lane];
         TileRes<R> res{R(0), R(0), R(0), R(0)};
         if (edge) tile_a_sweep<R, true, SH>(A, t, X, Ka, Kb, up, dn, rden_a, rden_b, res);
         else tile_a_sweep<R, false, SH>(A, t, X, Ka, Kb, up, dn, rden_a, rden_b, res);
@@ -624,6 +667,7 @@ __device__ __forceinline__ unsigned tile_a_sweeps(const ASweepArgs<R> *Ap, ATile
         bits |= __ballot(open) != 0ull ? 1u << s : 0u;
         __syncthreads();
     }
+    par_ = par;
     return bits;
 }
 
@@ -636,19 +680,39 @@ template <typename SH> __device__ __forceinline__ bool tile_ring_row(const TileC
     return tr < 2 * SH::H || tr >= SH::NW * SH::NR - 2 * SH::H;
 }
 
-// The tile's nodes (all of them, or just the ring) to a psi buffer.
+// The tile's nodes (all of them, or just the ring) to a psi buffer. `all` is
+// laundered: a copy of the code for each of its values would cost more in
+// instruction fetches, once a solve, than the lane masks do. The wait ahead
+// of the stores is for loads long past: without it the compiler waits, on
+// the common counter, ahead of every store (each value was once loaded on
+// some path), and the stores go out one at a time: 1.6 instead of 0.6 us for
+// the A links of 4 rows, and as long again until the last one is through.
 template <typename R, typename SH>
 __device__ __forceinline__ void tile_psi_publish(int Nx, int Ny, cplx<R> *out, const TileCtx &X0,
-                                                 const PsiTile<R, SH> &t, bool all) {
+                                                 const cplx<R> (&p)[SH::NR], bool all) {
     constexpr int NR = SH::NR, H = SH::H;
     const TileCtx X = X0.fresh();
-    const bool own = X.own<SH>(Nx), side = all || X.lane < 2 * H || X.lane >= WAVE - 2 * H;
+    const bool own = X.own<SH>(Nx), side = fresh_v(all) || X.lane < 2 * H || X.lane >= WAVE - 2 * H;
     const uint32_t cc = X.cc(Nx);
     const int r0 = X.r0<SH>(), r1 = X.r1<SH>(Ny);
+    __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
     for (int r = 0; r < NR; ++r)
         if (r >= r0 && r < r1 && own && (side || tile_ring_row<SH>(X, r)))
-            st_shared_mem(out + (size_t)Nx * (X.j0 + r) + cc, t.p[r]);
+            st_shared_mem(out + (size_t)Nx * (X.j0 + r) + cc, p[r]);
+}
+
+// psi^{n+1} = psi^n + D of a FP32 solve at the nodes of the tile.
+template <typename R, typename SH>
+__device__ __forceinline__ void tile_psi_total(int Nx, int Ny, const cplx<R> *psi, const TileCtx &X0,
+                                               const PsiTile<R, SH> &t, cplx<R> (&p)[SH::NR]) {
+    constexpr int NR = SH::NR;
+    const TileCtx X = X0.fresh();
+    const uint32_t oc = X.cc(Nx) * (uint32_t)sizeof(R);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) p[r] = ld_at(tile_row(psi, X.j0 + r, Ny, Nx), 2 * oc);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) p[r] = {p[r].re + t.rd[r].re, p[r].im + t.rd[r].im};
 }
 template <typename R, typename SH>
 __device__ __forceinline__ void tile_a_publish(int Nx, int Ny, R *out, const TileCtx &X0, const ATile<R, SH> &t,
@@ -657,9 +721,10 @@ __device__ __forceinline__ void tile_a_publish(int Nx, int Ny, R *out, const Til
     const TileCtx X = X0.fresh();
     const int Nxa = Nx - 1;
     R *out_b = out + (size_t)Nxa * Ny;
-    const bool own = X.own<SH>(Nx), side = all || X.lane < 2 * H || X.lane >= WAVE - 2 * H, hasa = X.hasa(Nx);
+    const bool own = X.own<SH>(Nx), side = fresh_v(all) || X.lane < 2 * H || X.lane >= WAVE - 2 * H, hasa = X.hasa(Nx);
     const uint32_t cc = X.cc(Nx);
     const int r0 = X.r0<SH>(), r1 = X.r1<SH>(Ny);
+    __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
     for (int r = 0; r < NR; ++r)
         if (r >= r0 && r < r1 && own && (side || tile_ring_row<SH>(X, r))) {
@@ -728,7 +793,7 @@ __device__ __forceinline__ bool tile_meet_neighbours(const TileSync &ts, const T
             ok = tile_poll(flag + (y - tm.ty) * tm.ntx + (x - tm.tx), epoch, ts.err, v) && ok;
         }
     }
-    return !__syncthreads_or(!ok);
+    return uniform(__syncthreads_or(!ok)) == 0;
 }
 
 // All workgroups of the instance meet: `bits` (per wave) are or-ed over all
@@ -781,8 +846,8 @@ __device__ __forceinline__ bool tile_meet_all(const TileSync &ts, const TileTeam
         }
     }
     __syncthreads();
-    out = S.all;
-    return S.fail == 0;
+    out = (unsigned)uniform((int)S.all);
+    return uniform(S.fail) == 0;
 }
 
 // ---- the run --------------------------------------------------------------------
@@ -819,55 +884,62 @@ struct TileSched {
 // the gauge-shifted form (link_phase).
 template <typename R, bool WITHA, typename SH>
 __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync &ts, const TileTeam &tm, int nsteps,
-                                         R thr_psi, R thr_a, int *st, int *sweeps, int stride, TileLds<R, SH> &S) {
+                                         R thr_psi, R thr_a, int *st, int *sweeps, int stride, bool passes, TileLds<R, SH> &S) {
     constexpr int NR = SH::NR, H = SH::H;
     constexpr bool GAUGE = WITHA && RunForm<R>::has_gauge;
     constexpr bool F64 = std::is_same<R, double>::value;
     constexpr int HA = H & ~1;  // A sweeps between exchanges: even, as the source changes with every second sweep
-    const int Nx = T->psi.Nx, Ny = T->psi.Ny;
+    const int Nx = arg(&T->psi.Nx), Ny = arg(&T->psi.Ny), max_sweeps = arg(&T->max_sweeps);
     const TileCtx X = tile_ctx<SH>(tm.tx, tm.ty);
+    if (X.w < 4)  // the rows of zeros; a barrier follows before any is read
+        S.edge[X.w >> 1][(X.w & 1) ? 2 * SH::NW + 1 : 0][X.lane] = {R(0), R(0)};
     PsiTile<R, SH> t;
-    int pc = st[ST_PSI], qc = st[ST_AB], pred = 0, pred_a = 0, par = 0;
+    int pc = uniform(st[ST_PSI]), qc = uniform(st[ST_AB]), pred = 0, pred_a = 0, par = 0;
     int redo = 0, redo_a = 0, done_steps = 0;
     unsigned long long ef = 0, ec = 0;  // epochs of the flag and check words
     bool ok = true;
     R rden_a = R(0), rden_b = R(0);
     if constexpr (F64 && WITHA) {
-        rden_a = R(1) / T->A.den_a;
-        rden_b = R(1) / T->A.den_b;
+        rden_a = R(1) / arg(&T->A.den_a);
+        rden_b = R(1) / arg(&T->A.den_b);
     }
     for (int step = 0; step < nsteps && ok; ++step) {
         // -- psi
         const int o1 = (pc + 1) % 3, o2 = (pc + 2) % 3;
         int cur = pc;  // the buffer published last
         {
-            if (WITHA || step == 0) tile_links<R, GAUGE, SH>(&T->psi, T->Q[qc], X, t);
-            TileSched sc(pred, H, T->max_sweeps);
+            if (WITHA || step == 0) tile_links<R, GAUGE, SH>(&T->psi, arg(&T->Q[uniform(qc)]), X, t);
+            TileSched sc(pred, H, max_sweeps);
             unsigned bits = 0u;
             int nsw = 0, stop = 0;  // stop: the sweep a redone solve ends at
             bool again;
+            cplx<R> tot[NR];  // psi^{n+1} (FP32)
             do {
                 again = false;
-                tile_psi_load<R, SH>(&T->psi, T->P[pc], X, t, S);
+                tile_psi_load<R, SH>(&T->psi, arg(&T->P[uniform(pc)]), X, t, S);
                 for (;;) {
                     par ^= 1;
                     tile_edges_out<R, SH>(S, par, X, t.p[0], t.p[NR - 1]);
                     __syncthreads();
-                    const int n = min(sc.next - sc.j, H);
-                    bits |= tile_psi_sweeps<R, SH>(&T->psi, t, S, X, n, thr_psi, par) << (sc.j - sc.j0);
+                    const int n = uniform(min(sc.next - sc.j, H));
+                    bits |= tile_psi_sweeps<R, SH>(&T->psi, t, S, X, n, thr_psi, par, uniform(sc.j) == 0) << (sc.j - sc.j0);
                     sc.j += n;
-                    const bool check = sc.j == sc.next;
+                    const bool check = uniform(sc.j) == uniform(sc.next);
                     cur = cur == o1 ? o2 : o1;
-                    tile_psi_publish<R, SH>(Nx, Ny, T->P[cur], X, t, check);
-                    if (!check) {
-                        if (!(ok = tile_meet_neighbours<R, SH>(ts, tm, ++ef, S))) break;
-                    } else {
+                    // FP32: all of psi^{n+1} goes out at a check, the ring of
+                    // changes where the solve goes on
+                    if (F64 || check) {
+                        if constexpr (!F64) tile_psi_total<R, SH>(Nx, Ny, arg(&T->P[uniform(pc)]), X, t, tot);
+                        const cplx<R>(&v)[NR] = F64 ? t.p : tot;
+                        tile_psi_publish<R, SH>(Nx, Ny, arg(&T->P[uniform(cur)]), X, v, check);
+                    }
+                    if (check) {
                         unsigned all = 0u;
                         if (!(ok = tile_meet_all<R, SH>(ts, tm, ++ec, S, bits, all))) break;
                         nsw = sc.j;
                         if (stop) break;  // a redone solve is over
                         const int m = sc.met(all);
-                        if (m == sc.j || (!m && sc.j >= T->max_sweeps)) break;
+                        if (m == sc.j || (!m && sc.j >= max_sweeps)) break;
                         bits = 0u;
                         if (m) {  // an earlier sweep met the stop rule: again from psi^n, up to that sweep
                             ++redo;
@@ -875,12 +947,21 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                             again = true;
                             break;
                         }
-                        sc.extend(pred, T->max_sweeps);
+                        sc.extend(pred, max_sweeps);
+                        if constexpr (!F64) cur = cur == o1 ? o2 : o1;
                     }
-                    tile_psi_halo<R, SH>(Nx, Ny, T->P[cur], X, t);
+                    if (!(F64 && check)) {
+                        if constexpr (!F64) tile_psi_publish<R, SH>(Nx, Ny, arg(&T->P[uniform(cur)]), X, t.p, false);
+                        if (!(ok = tile_meet_neighbours<R, SH>(ts, tm, ++ef, S))) break;
+                    }
+                    tile_psi_halo<R, SH>(Nx, Ny, arg(&T->P[uniform(cur)]), X, t);
                 }
             } while (again);
             if (!ok) break;
+            if constexpr (!F64) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) t.p[r] = tot[r];
+            }
             pred = nsw;
             if (threadIdx.x == 0 && tm.tx == 0 && tm.ty == 0) sweeps[(long)step * stride] = nsw;
         }
@@ -888,17 +969,16 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
         // -- A
         if constexpr (WITHA) {
             const int q1 = (qc + 1) % 3, q2 = (qc + 2) % 3;
-            const R *Q = T->Q[qc];
+            const R *Q = arg(&T->Q[uniform(qc)]);
             int qcur = qc;
             ATile<R, SH> u;
             // psi beyond the tile, and of the row below the wave's last one
-            tile_psi_halo<R, SH>(Nx, Ny, T->P[pc], X, t);
+            tile_psi_halo<R, SH>(Nx, Ny, arg(&T->P[uniform(pc)]), X, t);
             par ^= 1;
             tile_edges_out<R, SH>(S, par, X, t.p[0], t.p[NR - 1]);
             __syncthreads();
-            cplx<R> pdn = {R(0), R(0)};
-            if (!X.last<SH>()) pdn = S.edge[par][X.w + 1][0][X.lane];
-            TileSched sc(pred_a, HA, T->max_sweeps);
+            const cplx<R> pdn = S.edge[par][2 * X.w + 3][X.lane];
+            TileSched sc(pred_a, HA, max_sweeps);
             unsigned bits = 0u;
             int nsw = 0, stop = 0;
             bool again;
@@ -918,14 +998,14 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                     }
                     do {
                         if (sc.j % 2 == 0) tile_a_source<R, GAUGE, SH>(&T->A, t.p, t.ena, t.enb, pdn, Q, X, u);
-                        const int n = min(sc.next - sc.j, 2 - sc.j % 2);
+                        const int n = uniform(min(sc.next - sc.j, 2 - sc.j % 2));
                         bits |= tile_a_sweeps<R, SH>(&T->A, u, S, X, n, thr_a, par, rden_a, rden_b) << (sc.j - sc.j0);
                         sc.j += n;
                         seg += n;
                     } while (sc.j < sc.next && seg < HA);
-                    const bool check = sc.j == sc.next;
+                    const bool check = uniform(sc.j) == uniform(sc.next);
                     qcur = qcur == q1 ? q2 : q1;
-                    tile_a_publish<R, SH>(Nx, Ny, T->Q[qcur], X, u, check);
+                    tile_a_publish<R, SH>(Nx, Ny, arg(&T->Q[uniform(qcur)]), X, u, check);
                     if (!check) {
                         if (!(ok = tile_meet_neighbours<R, SH>(ts, tm, ++ef, S))) break;
                     } else {
@@ -934,7 +1014,7 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                         nsw = sc.j;
                         if (stop) break;
                         const int m = sc.met(all);
-                        if (m == sc.j || (!m && sc.j >= T->max_sweeps)) break;
+                        if (m == sc.j || (!m && sc.j >= max_sweeps)) break;
                         bits = 0u;
                         if (m) {
                             ++redo_a;
@@ -942,9 +1022,9 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                             again = true;
                             break;
                         }
-                        sc.extend(pred_a, T->max_sweeps);
+                        sc.extend(pred_a, max_sweeps);
                     }
-                    if (sc.j % 2 == 0) tile_a_halo<R, SH>(Nx, Ny, T->Q[qcur], X, u);
+                    if (sc.j % 2 == 0) tile_a_halo<R, SH>(Nx, Ny, arg(&T->Q[uniform(qcur)]), X, u);
                 }
             } while (again);
             if (!ok) break;
@@ -963,6 +1043,7 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
         }
         st[ST_PSI] = pc;
         st[ST_AB] = qc;
+        if (!passes) return;
         st[ST_PASS_PSI] = nsteps + redo;
         st[ST_REDO_PSI] = redo;
         st[ST_PASS_A] = WITHA ? nsteps + redo_a : 0;
@@ -978,7 +1059,7 @@ __global__ void __launch_bounds__(SH::NW * WAVE, 2)
     const TDSolveArgs<R> *T = (const TDSolveArgs<R> *)__builtin_amdgcn_kernarg_segment_ptr();
     const int wg = xcd_block();
     const TileTeam tm{0, 0, ntx * nty, wg % ntx, wg / ntx, ntx, nty};
-    tile_run<R, WITHA, SH>(T, ts, tm, nsteps, thr_psi, thr_a, T_.sc.state, T_.sc.sweeps, 2, S);
+    tile_run<R, WITHA, SH>(T, ts, tm, nsteps, thr_psi, thr_a, T_.sc.state, T_.sc.sweeps, 2, true, S);
 }
 
 }  // namespace glx

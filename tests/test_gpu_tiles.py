@@ -92,3 +92,16 @@ def test_tiles_equal_rows(size, kappa, dtype):
 ])
 def test_tile_schedules_equal_rows(dt, sigma, max_sweeps, eqn):
     compare(150, 131, np.float64, 5.0, True, 6, dt=dt, sigma=sigma, max_sweeps=max_sweeps, eqn=eqn)
+
+
+@pytest.mark.parametrize("kappa", [0.0, 5.0])
+@pytest.mark.parametrize("size", [(129, 129), (129, 513), (257, 65), (513, 257), (701, 690)])
+def test_fp32_tiles_stop_where_fp64_does(size, kappa):
+    # the FP32 tiles carry the changes themselves, to 1e-7 of their size, so
+    # the stop rule is met at the sweep where 64-bit iterates meet it (the
+    # difference of two FP32 iterates is off by up to 1e-1 of the rule)
+    f = state(*size, np.float32, True, seed=size[0] + 3 * size[1])
+    f64 = (f[0].astype(np.complex128), f[1].astype(np.float64), f[2], f[3].astype(np.float64))
+    sw = run(*size, np.float32, f, kappa, 0, 10)[2]
+    sw64 = run(*size, np.float64, f64, kappa, 8, 10)[2]
+    assert np.array_equal(sw[:, 0], sw64[:, 0])
