@@ -166,14 +166,16 @@ typedef struct glx_batch_instance {
     int32_t ab_cur;
 } glx_batch_instance;
 
-/* Advance n instances by nsteps TD steps. Every step is ONE persistent
- * launch in which each instance is swept by its own team of co-resident
- * workgroups with team-local barriers, so instances stop their Jacobi
- * solves independently (ragged sweep counts). Teams are sized in
- * proportion to each instance's wave-rows times weight[i] (its relative
- * sweeps per step, e.g. from an earlier run; NULL = 1). With use_graph != 0,
- * the step launches are captured once into a HIP graph and replayed.
- * wg_per_cu (co-resident workgroups per CU, 0 = as many as fit),
+/* Advance n instances by nsteps TD steps, each with its own stop rule and
+ * sweep counts (as glx_td_run would alone). Instances whose nodes fit in
+ * the registers of the GPU (up to about a million nodes) run all steps in
+ * one launch with as many others as fit beside them. For larger ones every
+ * step is ONE persistent launch in which each instance is swept by its own
+ * team of co-resident workgroups with team-local barriers; what follows is
+ * about these. Teams are sized in proportion to each instance's wave-rows
+ * times weight[i] (its relative sweeps per step, e.g. from an earlier run;
+ * NULL = 1). With use_graph != 0, the step launches are captured once into
+ * a HIP graph and replayed. wg_per_cu (co-resident workgroups per CU, 0 = as many as fit),
  * min_rows (fewest rows per wave when sizing teams, 0 = 16) and psi_depth
  * (sweeps per psi pass, 2..4, i.e. strips of 64 - 2*psi_depth columns;
  * 0 = 3) are the tunable tile shape; the results do not depend on them.

@@ -2,13 +2,14 @@
 
 The reference runs one GLSolver per process, one time step at a time
 (svirl/solvers/td.py:342-366). Here a list of solvers of the same precision
-(each with its own grid, kappa, field, epsilon map and mask) advances by one
-persistent launch per time step (glx_batch_td_run): every instance is swept
-by its own team of workgroups with team-local barriers, so each instance
-keeps its own Jacobi sweep counts and stop rule, exactly as if it had been
-run alone. The step launches are replayed from a captured HIP graph.
+(each with its own grid, kappa, field, epsilon map and mask) advances
+together (glx_batch_td_run): every instance is swept by its own workgroups,
+so each keeps its own Jacobi sweep counts and stop rule, exactly as if it had
+been run alone. Instances of up to about a million nodes are held in
+registers and run all steps in one launch, as many at a time as fit.
 
-The tile shape — sweeps per psi pass (the tile depth, which sets the
+Larger ones advance by one persistent launch per time step, replayed from a
+captured HIP graph, in teams of workgroups whose shape matters. That shape — sweeps per psi pass (the tile depth, which sets the
 strip width: 64 - 2 x depth columns per wave), fewest rows per wave when
 sizing the teams (the tile height) and workgroups per CU — is picked by an
 autotuner: the first steps of a run time candidate shapes on the real state

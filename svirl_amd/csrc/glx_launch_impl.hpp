@@ -639,7 +639,7 @@ template <typename R, bool G, int KB> static int batch_occupancy(int *per_cu) {
 template <typename R, bool G, int KB>
 static int batch_run_form(const Env &e, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
                           int32_t use_graph, int32_t wg_per_cu, int32_t min_rows, const double *weight,
-                          const Workspace &ws) {
+                          const Workspace &ws, bool check_only) {
     int per_cu = 0;
     int rc = batch_occupancy<R, G, KB>(&per_cu);
     if (rc) return rc;
@@ -682,7 +682,9 @@ static int batch_run_form(const Env &e, glx_batch_instance *inst, int32_t n, int
             return set_error(GLX_E_ARG, "%s: %d instances x %d steps need %zu bytes of scratch, above its %zu-byte maximum",
                              ws.what, n, nsteps, need, ws.bytes);
         blk = (char *)ws.ptr;
-    } else {
+    }
+    if (check_only) return GLX_OK;
+    if (!ws.ptr) {
         st = hipMalloc((void **)&blk, need);
         if (st != hipSuccess) return check_hip(st, "hipMalloc(batch)");
     }
@@ -775,6 +777,232 @@ static int batch_run_form(const Env &e, glx_batch_instance *inst, int32_t n, int
     return GLX_OK;
 }
 
+// ---- batches on register tiles -----------------------------------------------------
+
+// The co-resident workgroups of the batch's tile kernel, queried once.
+template <typename R, bool WITHA, typename SH> static int batch_tile_capacity(const Env &e, long *cap) {
+    static int per_cu = 0;
+    if (per_cu <= 0) {
+        int m = 0;
+        hipError_t st = hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, k_batch_td_tiles<R, WITHA, SH>, SH::NW * WAVE, 0);
+        if (st != hipSuccess) return check_hip(st, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+        per_cu = m;
+    }
+    *cap = std::min((long)per_cu * e.num_cus, (long)MAX_GRID_BLOCKS);
+    return GLX_OK;
+}
+
+// One launch of a batch: a tile shape and the instances whose tiles are
+// resident together.
+struct TileBin {
+    int shape, used;
+    std::vector<TileInst> inst;
+};
+
+// Launches for the instances `todo` (all with or all without an A solve),
+// largest first into the first launch with room. The shape is the one whose
+// launches cost least (tile_cost of each); instances that do not fit it go
+// to a larger one the same way. Returns the cost; `bins` and `left` (those
+// no shape holds) are appended to.
+template <typename R, bool WITHA>
+static int plan_tile_bins(const Env &e, const glx_batch_instance *inst, const std::vector<int> &todo, double *cost,
+                          std::vector<TileBin> &bins, std::vector<int> &left) {
+    using Shapes = typename TileShapes<R>::list;
+    *cost = 0.0;
+    if (todo.empty()) return GLX_OK;
+    int rc = GLX_OK;
+    bool found = false;
+    std::vector<TileBin> best_bins;
+    std::vector<int> best_left;
+    each_shape<Shapes>([&](auto k) {
+        using T = std::tuple_element_t<k, Shapes>;
+        long cap = 0;
+        if (!rc) rc = batch_tile_capacity<R, WITHA, T>(e, &cap);
+        if (rc) return;
+        std::vector<TileBin> mine;
+        std::vector<int> rest, order = todo;
+        auto tiles = [&](int i) {
+            return (long)((inst[i].g.Nx + T::COLS - 1) / T::COLS) * ((inst[i].g.Ny + T::ROWS - 1) / T::ROWS);
+        };
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return tiles(a) > tiles(b); });
+        for (int i : order) {
+            const long t = tiles(i);
+            if (t > cap) {
+                rest.push_back(i);
+                continue;
+            }
+            size_t q = 0;
+            while (q < mine.size() && mine[q].used + t > cap) ++q;
+            if (q == mine.size()) mine.push_back({(int)k, 0, {}});
+            TileInst I{};
+            I.b0 = mine[q].used;
+            I.ntx = (inst[i].g.Nx + T::COLS - 1) / T::COLS;
+            I.nty = (inst[i].g.Ny + T::ROWS - 1) / T::ROWS;
+            I.id = i;
+            mine[q].inst.push_back(I);
+            mine[q].used += (int)t;
+        }
+        if (mine.empty()) return;
+        double c = 0.0;
+        for (const TileBin &b : mine) c += tile_cost<T>(e, TilePlan{b.used, 1, true});
+        double more = 0.0;
+        std::vector<int> none;
+        if (!rest.empty()) rc = plan_tile_bins<R, WITHA>(e, inst, rest, &more, mine, none);
+        if (rc) return;
+        // leaving instances to the row-marching teams is the last resort
+        c += more + 1.0e6 * (double)none.size();
+        if (!found || c < *cost) {
+            found = true;
+            *cost = c;
+            best_bins = std::move(mine);
+            best_left = std::move(none);
+        }
+    });
+    if (rc) return rc;
+    if (!found) {
+        left.insert(left.end(), todo.begin(), todo.end());
+        return GLX_OK;
+    }
+    bins.insert(bins.end(), best_bins.begin(), best_bins.end());
+    left.insert(left.end(), best_left.begin(), best_left.end());
+    return GLX_OK;
+}
+
+// Zero the words of one launch's tiles; the error flag is set with the
+// batch's first launch (err0 >= 0) only.
+static __global__ void k_batch_tile_reset(TileSync ts, int nwg, int ngrp, int err0) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nwg) ts.flag[k] = ts.chk[0][k] = ts.chk[1][k] = 0ull;
+    if (k < ngrp) ts.grp[0][k] = ts.grp[1][k] = 0ull;
+    if (k == 0 && err0 >= 0) *ts.err = err0;
+}
+
+// The instances of a batch that fit a tile shape, in launches of those that
+// fit together, each running all steps; `left`: the others. 32 FP32 grids
+// of 65 to 1025 nodes a side, 10 steps: 9.9 ms a call on row-marching teams
+// (one launch a step, a team's passes bound by their slowest row chain), 6.1
+// here, in five launches bound by their largest instances.
+template <typename R>
+static int batch_run_tiles(const Env &e, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
+                           const Workspace &ws, std::vector<int> *left) {
+    constexpr bool G = RunForm<R>::has_gauge;
+    std::vector<TileBin> bins[2];  // without, with A
+    std::vector<int> todo[2];
+    for (int i = 0; i < n; ++i) todo[inst[i].p.solveA ? 1 : 0].push_back(i);
+    double cost = 0.0;
+    int rc = plan_tile_bins<R, false>(e, inst, todo[0], &cost, bins[0], *left);
+    if (!rc) rc = plan_tile_bins<R, true>(e, inst, todo[1], &cost, bins[1], *left);
+    if (rc || (bins[0].empty() && bins[1].empty())) return rc;
+    std::vector<TDSolveArgs<R>> args(n);
+    std::vector<int> state(8 * (size_t)n, 0);
+    for (int i = 0; i < n; ++i) {
+        args[i] = batch_args<R>(inst[i], G);
+        state[8 * i + ST_PSI] = inst[i].psi_cur;
+        state[8 * i + ST_AB] = inst[i].ab_cur;
+    }
+    for (int i : *left) args[i].solveA = 0;  // not this launch's to shift
+    std::vector<TileInst> table;
+    for (auto &side : bins)
+        for (TileBin &b : side) {
+            int g = 0;
+            for (TileInst &I : b.inst) {
+                I.gbase = g;
+                g += (I.ntx * I.nty + TILE_GROUP - 1) / TILE_GROUP;
+                I.thr_psi = (double)stop_threshold<R>(args[I.id].psi.stop_eps);
+                I.thr_a = (double)stop_threshold<R>(args[I.id].A.stop_eps);
+                table.push_back(I);
+            }
+        }
+    // one device block: args | table | state | sweeps, smaller than the
+    // row-marching teams' for the same batch
+    auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t s_args = al(sizeof(TDSolveArgs<R>) * n), s_table = al(sizeof(TileInst) * table.size());
+    const size_t s_state = al(sizeof(int) * 8 * n), s_sw = al(sizeof(int) * 2 * (size_t)n * nsteps);
+    const size_t need = s_args + s_table + s_state + s_sw;
+    char *blk = (char *)ws.ptr;
+    if (ws.ptr && need > ws.bytes)
+        return set_error(GLX_E_ARG, "%s: %d instances x %d steps need %zu bytes of scratch, above its %zu-byte maximum",
+                         ws.what, n, nsteps, need, ws.bytes);
+    hipError_t st = hipSuccess;
+    if (!ws.ptr) {
+        st = hipMalloc((void **)&blk, need);
+        if (st != hipSuccess) return check_hip(st, "hipMalloc(batch)");
+    }
+    struct Free { char *p; ~Free() { if (p) (void)hipFree(p); } } guard{ws.ptr ? nullptr : blk};
+    TDSolveArgs<R> *d_args = (TDSolveArgs<R> *)blk;
+    TileInst *d_table = (TileInst *)(blk + s_args);
+    int *d_state = (int *)(blk + s_args + s_table), *d_sw = (int *)(blk + s_args + s_table + s_state);
+    st = hipMemcpyAsync(d_args, args.data(), sizeof(TDSolveArgs<R>) * n, hipMemcpyHostToDevice, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(d_table, table.data(), sizeof(TileInst) * table.size(), hipMemcpyHostToDevice, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(d_state, state.data(), sizeof(int) * 8 * n, hipMemcpyHostToDevice, e.stream);
+    if (st != hipSuccess) return check_hip(st, "glx_batch_td_run upload");
+    long most = 1;
+    for (int i = 0; i < n; ++i) most = std::max(most, 2L * inst[i].g.Nx * inst[i].g.Ny);
+    auto shift = [&](double sign) {
+        if (!G || bins[1].empty()) return (int)GLX_OK;
+        hipLaunchKernelGGL(k_batch_gauge_shift<R>, dim3(grid_blocks(most, 1024, 256), n), dim3(256), 0, e.stream,
+                           (const TDSolveArgs<R> *)d_args, (const int *)d_state, sign);
+        GLX_LAUNCH_CHECK("k_batch_gauge_shift");
+        return (int)GLX_OK;
+    };
+    rc = shift(-1.0);
+    if (rc) return rc;
+    st = hipEventRecord(e.kev0, e.stream);
+    if (st != hipSuccess) return check_hip(st, "hipEventRecord");
+    const TileSync ts = tile_sync(e);
+    int err0 = e.abort_next ? 1 : 0;
+    const TileInst *t = d_table;
+    auto launch = [&](auto withA, const std::vector<TileBin> &side) -> int {
+        using Shapes = typename TileShapes<R>::list;
+        for (const TileBin &b : side) {
+            const TileInst &z = b.inst.back();
+            const int ngrp = z.gbase + (z.ntx * z.nty + TILE_GROUP - 1) / TILE_GROUP;
+            hipLaunchKernelGGL(k_batch_tile_reset, dim3((std::max(b.used, ngrp) + 255) / 256), dim3(256), 0, e.stream, ts,
+                               b.used, ngrp, err0);
+            GLX_LAUNCH_CHECK("k_batch_tile_reset");
+            err0 = -1;
+            each_shape<Shapes>([&](auto k) {
+                using T = std::tuple_element_t<k, Shapes>;
+                if ((int)k == b.shape)
+                    hipLaunchKernelGGL((k_batch_td_tiles<R, decltype(withA)::value, T>), dim3(b.used), dim3(T::NW * WAVE),
+                                       0, e.stream, (const TDSolveArgs<R> *)d_args, t, (int)b.inst.size(), ts, d_state,
+                                       d_sw, (int)n, (int)nsteps);
+            });
+            GLX_LAUNCH_CHECK("k_batch_td_tiles");
+            t += b.inst.size();
+        }
+        return GLX_OK;
+    };
+    rc = launch(std::false_type{}, bins[0]);
+    if (!rc) rc = launch(std::true_type{}, bins[1]);
+    if (rc) return rc;
+    st = hipEventRecord(e.kev1, e.stream);
+    if (st != hipSuccess) return check_hip(st, "hipEventRecord");
+    rc = shift(1.0);
+    if (rc) return rc;
+    int host_err = 0;
+    std::vector<int> sw(sweeps ? 2 * (size_t)n * nsteps : 0);
+    st = hipMemcpyAsync(state.data(), d_state, sizeof(int) * 8 * n, hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(&host_err, e.err, sizeof(int), hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess && sweeps)
+        st = hipMemcpyAsync(sw.data(), d_sw, sizeof(int) * sw.size(), hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
+    if (st != hipSuccess) return check_hip(st, "glx_batch_td_run readback");
+    float kms = 0.f;
+    if (hipEventElapsedTime(&kms, e.kev0, e.kev1) == hipSuccess && e.last_kernel_ms) *e.last_kernel_ms = kms;
+    if (host_err) return set_error(GLX_E_TIMEOUT, "%s: a team barrier timed out", ws.what);
+    std::vector<char> mine(n, 1);
+    for (int i : *left) mine[i] = 0;
+    for (int i = 0; i < n; ++i) {
+        if (!mine[i]) continue;
+        inst[i].psi_cur = state[8 * i + ST_PSI];
+        inst[i].ab_cur = state[8 * i + ST_AB];
+        for (int j = 0; sweeps && j < nsteps; ++j)
+            for (int q = 0; q < 2; ++q) sweeps[2 * ((size_t)j * n + i) + q] = sw[2 * ((size_t)j * n + i) + q];
+    }
+    return GLX_OK;
+}
+
 template <typename R>
 int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
                        int32_t use_graph, int32_t wg_per_cu, int32_t min_rows, const double *weight,
@@ -801,18 +1029,48 @@ int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_
         any_A = any_A || p.solveA;
     }
     if (nsteps == 0) return GLX_OK;
-    auto run = [&](auto g, auto kb) {
-        return batch_run_form<R, decltype(g)::value, decltype(kb)::value>(e, inst, n, nsteps, sweeps, use_graph,
-                                                                         wg_per_cu, min_rows, weight, ws);
+    // instances on the row-marching teams (all of them: check only)
+    auto rows = [&](glx_batch_instance *in, int32_t m, int32_t *sw, const double *wt, bool check_only) {
+        auto run = [&](auto g, auto kb) {
+            return batch_run_form<R, decltype(g)::value, decltype(kb)::value>(e, in, m, nsteps, sw, use_graph, wg_per_cu,
+                                                                             min_rows, wt, ws, check_only);
+        };
+        auto by_depth = [&](auto g) {
+            if (psi_depth == 2) return run(g, std::integral_constant<int, 2>{});
+            if (psi_depth == 4) return run(g, std::integral_constant<int, 4>{});
+            return run(g, std::integral_constant<int, 3>{});
+        };
+        if constexpr (RunForm<R>::has_gauge)
+            if (any_A) return by_depth(std::true_type{});
+        return by_depth(std::false_type{});
     };
-    auto by_depth = [&](auto g) {
-        if (psi_depth == 2) return run(g, std::integral_constant<int, 2>{});
-        if (psi_depth == 4) return run(g, std::integral_constant<int, 4>{});
-        return run(g, std::integral_constant<int, 3>{});
-    };
-    if constexpr (RunForm<R>::has_gauge)
-        if (any_A) return by_depth(std::true_type{});
-    return by_depth(std::false_type{});
+    // what the teams would refuse (too many instances, too little scratch) is refused
+    int rc = rows(inst, n, nullptr, weight, true);
+    if (rc) return rc;
+    std::vector<int> left;
+    rc = batch_run_tiles<R>(e, inst, n, nsteps, sweeps, ws, &left);
+    if (rc || left.empty()) return rc;
+    if ((int)left.size() == n) return rows(inst, n, sweeps, weight, false);
+    // the instances no tile shape holds
+    const int m = (int)left.size();
+    std::vector<glx_batch_instance> sub(m);
+    std::vector<double> wt(weight ? m : 0);
+    std::vector<int32_t> sw(sweeps ? 2 * (size_t)m * nsteps : 0);
+    for (int k = 0; k < m; ++k) {
+        sub[k] = inst[left[k]];
+        if (weight) wt[k] = weight[left[k]];
+    }
+    const float ms = e.last_kernel_ms ? *e.last_kernel_ms : 0.f;
+    rc = rows(sub.data(), m, sweeps ? sw.data() : nullptr, weight ? wt.data() : nullptr, false);
+    if (rc) return rc;
+    if (e.last_kernel_ms) *e.last_kernel_ms += ms;
+    for (int k = 0; k < m; ++k) {
+        inst[left[k]].psi_cur = sub[k].psi_cur;
+        inst[left[k]].ab_cur = sub[k].ab_cur;
+        for (int j = 0; sweeps && j < nsteps; ++j)
+            for (int q = 0; q < 2; ++q) sweeps[2 * ((size_t)j * n + left[k]) + q] = sw[2 * ((size_t)j * m + k) + q];
+    }
+    return GLX_OK;
 }
 
 // ---- batched CG -----------------------------------------------------------------

@@ -1905,9 +1905,11 @@ static __global__ void k_td_reset(TDScratch sc, int pc, int qc, int err0) {
     }
 }
 
-// A <-> A - A_g on every link, in place (sign -1: remove, +1: add back).
+// A <-> A - A_g on every link, in place (sign -1: remove, +1: add back), by
+// the workgroups of the launch's first dimension.
 template <typename R>
-__global__ void k_gauge_shift(R *ab, int Nx, int Ny, double H, double dx, double dy, double x0, double y0, double sign) {
+__device__ __forceinline__ void gauge_shift(R *ab, int Nx, int Ny, double H, double dx, double dy, double x0, double y0,
+                                            double sign) {
     const long Na = (long)(Nx - 1) * Ny, Nab = Na + (long)Nx * (Ny - 1);
     for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < Nab; k += (long)gridDim.x * blockDim.x) {
         double g;
@@ -1916,20 +1918,17 @@ __global__ void k_gauge_shift(R *ab, int Nx, int Ny, double H, double dx, double
         ab[k] = R(double(ab[k]) + sign * g);
     }
 }
+template <typename R>
+__global__ void k_gauge_shift(R *ab, int Nx, int Ny, double H, double dx, double dy, double x0, double y0, double sign) {
+    gauge_shift<R>(ab, Nx, Ny, H, dx, dy, x0, y0, sign);
+}
 
-// k_gauge_shift on the buffer holding the run's current vector potential.
+// gauge_shift on the buffer holding the run's current vector potential.
 template <typename R>
 __global__ void k_gauge_shift_state(R *q0, R *q1, R *q2, const int *state, int Nx, int Ny, double H, double dx,
                                     double dy, double x0, double y0, double sign) {
     const int k = state[ST_AB];
-    R *ab = k == 0 ? q0 : (k == 1 ? q1 : q2);
-    const long Na = (long)(Nx - 1) * Ny, Nab = Na + (long)Nx * (Ny - 1);
-    for (long n = blockIdx.x * (long)blockDim.x + threadIdx.x; n < Nab; n += (long)gridDim.x * blockDim.x) {
-        double g;
-        if (n < Na) g = gauge_a(H, dy, y0, (int)(n / (Nx - 1)));
-        else g = gauge_b(H, dx, x0, (int)((n - Na) % Nx));
-        ab[n] = R(double(ab[n]) + sign * g);
-    }
+    gauge_shift<R>(k == 0 ? q0 : (k == 1 ? q1 : q2), Nx, Ny, H, dx, dy, x0, y0, sign);
 }
 
 }  // namespace glx

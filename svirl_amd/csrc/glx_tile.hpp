@@ -1062,4 +1062,41 @@ __global__ void __launch_bounds__(SH::NW * WAVE, 2)
     tile_run<R, WITHA, SH>(T, ts, tm, nsteps, thr_psi, thr_a, T_.sc.state, T_.sc.sweeps, 2, true, S);
 }
 
+// A batch: the tiles of many instances in one launch, each instance with
+// its own words, state and sweep counts. Instance k of the launch has the
+// workgroups from inst[k].b0 on; where its arguments, state and sweeps lie
+// is numbered by inst[k].id.
+struct TileInst {
+    int b0, ntx, nty, gbase, id, pad;
+    double thr_psi, thr_a;
+};
+
+template <typename R, bool WITHA, typename SH>
+__global__ void __launch_bounds__(SH::NW * WAVE, 2)
+    k_batch_td_tiles(const TDSolveArgs<R> *args, const TileInst *inst, int ninst, TileSync ts, int *state, int *sweeps,
+                     int n, int nsteps) {
+    __shared__ TileLds<R, SH> S;
+    const int wg = xcd_block();
+    int lo = 0, hi = ninst;  // the last instance that begins at or before wg
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (arg(&inst[mid].b0) <= wg) lo = mid;
+        else hi = mid;
+    }
+    const TileInst I = fresh_args(inst + lo);
+    const int local = wg - I.b0;
+    const TileTeam tm{I.b0, I.gbase, I.ntx * I.nty, local % I.ntx, local / I.ntx, I.ntx, I.nty};
+    tile_run<R, WITHA, SH>(args + I.id, ts, tm, nsteps, R(I.thr_psi), R(I.thr_a), state + 8 * I.id,
+                           sweeps + 2 * I.id, 2 * n, false, S);
+}
+
+// A <-> A - A_g of the batch's instances that evolve A (args[k].solveA), one
+// row of workgroups each; the buffer is the one the state says.
+template <typename R> __global__ void __launch_bounds__(256) k_batch_gauge_shift(const TDSolveArgs<R> *args, const int *state, double sign) {
+    const int k = blockIdx.y;
+    const TDSolveArgs<R> &T = args[k];
+    if (!T.solveA) return;
+    gauge_shift<R>(pick3(T.Q, state[8 * k + ST_AB]), T.A.Nx, T.A.Ny, T.A.gH, T.A.gdx, T.A.gdy, T.A.gx0, T.A.gy0, sign);
+}
+
 }  // namespace glx

@@ -105,3 +105,49 @@ def test_fp32_tiles_stop_where_fp64_does(size, kappa):
     sw = run(*size, np.float32, f, kappa, 0, 10)[2]
     sw64 = run(*size, np.float64, f64, kappa, 8, 10)[2]
     assert np.array_equal(sw[:, 0], sw64[:, 0])
+
+
+def run_batch(insts, dtype, nsteps, noalloc):
+    """[(Nx, Ny, kappa, fields)] advanced together; (psi, ab, sweeps) of each."""
+    up = nat.DeviceArray.from_host
+    arr = (nat.BatchInstance * len(insts))()
+    bufs = []
+    for I, (Nx, Ny, kappa, (psi, ab, mt, eps)) in zip(arr, insts):
+        P = [up(psi)] + [nat.DeviceArray.zeros(psi.size, psi.dtype) for _ in range(2)]
+        Q = [up(ab)] + [nat.DeviceArray.zeros(ab.size, ab.dtype) for _ in range(2)]
+        d_mt, d_eps = (None if v is None else up(v) for v in (mt, eps))
+        bufs.append((P, Q, d_mt, d_eps))
+        I.g = nat.Grid(Nx, Ny, 0.5, 0.5)
+        prm = I.p
+        prm.dt, prm.eps, prm.kappa2, prm.rho, prm.H = 0.1, 0.0 if eps is not None else 1.0, kappa * kappa, 0.005, H
+        prm.stop_psi = prm.stop_A = 1e-6
+        prm.rand_t, prm.solveA, prm.max_sweeps, prm.eqn = 1, 1 if kappa else 0, 1024, 0
+        I.eps_map, I.mt = nat.ptr(d_eps), nat.ptr(d_mt)
+        for j in range(3):
+            I.psi[j], I.ab[j] = P[j].ptr, Q[j].ptr
+        I.psi_cur = I.ab_cur = 0
+    n = len(insts)
+    sw = (ctypes.c_int32 * (2 * n * nsteps))()
+    if noalloc:
+        nat.call("glx_batch_td_run_noalloc", nat.prec_of(dtype), arr, n, nsteps, sw, 0, 0, None, 0)
+    else:
+        nat.call("glx_batch_td_run", nat.prec_of(dtype), arr, n, nsteps, sw, 0, 0, 0, None, 0)
+    sw = np.frombuffer(sw, dtype=np.int32).reshape(nsteps, n, 2)
+    return [(b[0][I.psi_cur].get(), b[1][I.ab_cur].get(), sw[:, k].copy()) for k, (I, b) in enumerate(zip(arr, bufs))]
+
+
+# one instance; many small ones, with and without A; more tiles than one
+# launch holds; one grid that no tile shape holds among ones that fit
+BATCHES = [[(57, 9)], [(4, 4), (33, 70), (130, 65), (56, 24), (5, 300)] * 5, [(400, 500)] * 6 + [(65, 65)],
+           [(1100, 1100), (129, 257), (1100, 1100), (64, 64)]]
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+def test_batch_on_tiles_equals_rows(batch, noalloc):
+    sizes = BATCHES[batch]
+    insts = [(*s, 0.0 if k % 3 == 1 else 5.0, state(*s, np.float64, k % 2 == 0, seed=k)) for k, s in enumerate(sizes)]
+    for (psi, ab, sw), (Nx, Ny, kappa, f) in zip(run_batch(insts, np.float64, 3, noalloc), insts):
+        psi1, ab1, sw1 = run(Nx, Ny, np.float64, f, kappa, 8, 3)
+        assert np.array_equal(sw, sw1)
+        assert np.array_equal(psi, psi1) and np.array_equal(ab, ab1)
