@@ -41,33 +41,46 @@ enum {
     CG_IT0 = 8, CG_MARK = 9, CG_SINCE = 10, CG_NSTATE = 12
 };
 
-// Sum of L doubles per thread over the workgroup, into out (thread 0).
-template <int L> __device__ __forceinline__ void block_sums(double (&acc)[L], double *lds, double *out) {
+// Sums of L doubles per thread over the workgroup of NW waves, into out;
+// `part` holds L * NW doubles.
+template <int L, int NW>
+__device__ __forceinline__ void block_sums(const double (&acc)[L], double (&part)[L][NW], double *out) {
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
 #pragma unroll
     for (int k = 0; k < L; ++k) {
-        const double s = block_sum(acc[k], lds);
-        if (threadIdx.x == 0) out[k] = s;
-        __syncthreads();
+        const double s = wave_sum(acc[k]);
+        if (lane == 0) part[k][wid] = s;
     }
+    __syncthreads();
+    if (threadIdx.x < L) {
+        double s = 0.0;
+        for (int w = 0; w < NW; ++w) s += part[threadIdx.x][w];
+        out[threadIdx.x] = s;
+    }
+    __syncthreads();
 }
 
-// FP32: at most 128 VGPRs, so that four workgroups share a CU and a
-// 1024-instance batch is resident at once on 256 CUs (at the 164 the
-// kernel would otherwise take, three fit and a launch runs in two rounds).
-// FP64 keeps the default bound (capping it spills the line search).
-template <typename R> struct BatchCGBound { static constexpr int MIN_WG = 1; };
-template <> struct BatchCGBound<float> { static constexpr int MIN_WG = 4; };
+// The threads of an instance's workgroup: as many as fill the registers of
+// the CUs with the batch's instances resident together. A wave waits out the
+// memory latency of its nodes' loads, so an instance alone on a CU with the
+// four waves of a full batch leaves the CU idle most of the time: 256
+// instances of 129 x 129 (FP32, kappa < inf), per iteration: 718 us with 4
+// waves, 420 with 8, 306 with 16, of which 42 move the update at the rate of
+// the memory. FP32 stays below 128 VGPRs (16 waves a CU; 1024
+// instances are resident at 4 waves each), FP64 below 256 (8 waves).
+template <typename R> struct BatchCGWaves { static constexpr int PER_CU = 8; };
+template <> struct BatchCGWaves<float> { static constexpr int PER_CU = 16; };
 
 // Stall rule (stall_iters > 0): an instance whose relative gradient norm
 // has not halved within stall_iters iterations stops with flag 2 (the
 // FP32-mixed form stalls at the resolution of its gradient).
-template <typename R, int L>
-__global__ void __launch_bounds__(256, BatchCGBound<R>::MIN_WG) k_batch_cg(const CGInst<R> *insts, double *state, int n, int iters,
-                                                  int max_iters, double rtol, int stall_iters) {
-    __shared__ double lds[8];
+template <typename R, int L, int NW>
+__global__ void __launch_bounds__(NW * WAVE, BatchCGWaves<R>::PER_CU / NW)
+    k_batch_cg(const CGInst<R> *insts, double *state, int n, int iters, int max_iters, double rtol, int stall_iters) {
+    __shared__ double lds[NW], part[L][NW], part5[5][NW];
     __shared__ double red[L];
     __shared__ double bc[4];   // beta_psi, beta_A, alpha_psi, alpha_A
-    __shared__ int go, s_it;
+    __shared__ int go, s_it, s_first;
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
         const CGInst<R> &I = insts[k];
         const Geo &g = I.g;
@@ -79,18 +92,22 @@ __global__ void __launch_bounds__(256, BatchCGBound<R>::MIN_WG) k_batch_cg(const
             if (threadIdx.x == 0) {
                 go = (sv[CG_DONE] == 0.0 && sv[CG_IT] < (double)max_iters) ? 1 : 0;
                 s_it = (int)sv[CG_IT];
+                s_first = sv[CG_IT] == sv[CG_IT0] ? 1 : 0;
             }
             __syncthreads();
             if (!go) break;
             const int itn = s_it;
+            const bool first = s_first != 0;
             // (selects, not indexing: a run-time index into the instance
             // record would move the whole record to scratch memory)
             const bool odd = (itn & 1) != 0;
             cplx<R> *jac = odd ? I.jac[1] : I.jac[0], *jprev = odd ? I.jac[0] : I.jac[1];
             R *jacA = odd ? I.jacA[1] : I.jacA[0], *jprevA = odd ? I.jacA[0] : I.jacA[1];
-            // the direction of the previous iteration and this iteration's
-            cplx<R> *dold = odd ? I.dir[1] : I.dir[0], *dnew = odd ? I.dir[0] : I.dir[1];
-            R *dAold = odd ? I.dirA[1] : I.dirA[0], *dAnew = odd ? I.dirA[0] : I.dirA[1];
+            // the direction of the previous iteration (any finite values with
+            // the first iteration's beta of zero: the scratch arrays start
+            // out unwritten) and this iteration's
+            cplx<R> *dold = first ? jac : (odd ? I.dir[1] : I.dir[0]), *dnew = odd ? I.dir[0] : I.dir[1];
+            R *dAold = first ? jacA : (odd ? I.dirA[1] : I.dirA[0]), *dAnew = odd ? I.dirA[0] : I.dirA[1];
             // 1. gradients, PR sums and the gradient norm
             double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // |g|^2, num_psi, den_psi, num_A, den_A
             for (long m = threadIdx.x; m < g.N; m += blockDim.x) {
@@ -126,7 +143,7 @@ __global__ void __launch_bounds__(256, BatchCGBound<R>::MIN_WG) k_batch_cg(const
                     }
                 }
             }
-            block_sums<5>(acc, lds, red);
+            block_sums<5, NW>(acc, part5, red);
             if (threadIdx.x == 0) {
                 const double gn = sqrt(red[0]);
                 const int it0 = (int)sv[CG_IT0];
@@ -174,7 +191,7 @@ __global__ void __launch_bounds__(256, BatchCGBound<R>::MIN_WG) k_batch_cg(const
 #pragma unroll
                 for (int c = 0; c < L; ++c) cacc[c] += double(C[c]);
             }
-            block_sums<L>(cacc, lds, red);
+            block_sums<L, NW>(cacc, part, red);
             th = block_max(th, lds);
             th = __shfl(th, 0, WAVE);  // block_max leaves it in thread 0
             if (threadIdx.x < WAVE) {  // the first wave runs the line search

@@ -918,11 +918,17 @@ static int batch_run_tiles(const Env &e, glx_batch_instance *inst, int32_t n, in
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t s_args = al(sizeof(TDSolveArgs<R>) * n), s_table = al(sizeof(TileInst) * table.size());
     const size_t s_state = al(sizeof(int) * 8 * n), s_sw = al(sizeof(int) * 2 * (size_t)n * nsteps);
-    const size_t need = s_args + s_table + s_state + s_sw;
-    char *blk = (char *)ws.ptr;
+    // and, in a block of its own, the words the tiles meet by: calls of
+    // several threads run one after the other on the stream, each with its own
+    size_t nwords = 0;
+    for (auto &side : bins)
+        for (const TileBin &b : side) nwords = std::max(nwords, (size_t)b.used + b.inst.size());
+    const size_t s_words = ws.ptr ? 0 : al(8 * (5 * nwords + 1));
+    const size_t need = s_args + s_table + s_state + s_sw + s_words;
     if (ws.ptr && need > ws.bytes)
         return set_error(GLX_E_ARG, "%s: %d instances x %d steps need %zu bytes of scratch, above its %zu-byte maximum",
                          ws.what, n, nsteps, need, ws.bytes);
+    char *blk = (char *)ws.ptr;
     hipError_t st = hipSuccess;
     if (!ws.ptr) {
         st = hipMalloc((void **)&blk, need);
@@ -949,7 +955,11 @@ static int batch_run_tiles(const Env &e, glx_batch_instance *inst, int32_t n, in
     if (rc) return rc;
     st = hipEventRecord(e.kev0, e.stream);
     if (st != hipSuccess) return check_hip(st, "hipEventRecord");
-    const TileSync ts = tile_sync(e);
+    TileSync ts = tile_sync(e);
+    if (!ws.ptr) {
+        unsigned long long *w = (unsigned long long *)(blk + s_args + s_table + s_state + s_sw);
+        ts = TileSync{w, {w + nwords, w + 2 * nwords}, {w + 3 * nwords, w + 4 * nwords}, (int *)(w + 5 * nwords)};
+    }
     int err0 = e.abort_next ? 1 : 0;
     const TileInst *t = d_table;
     auto launch = [&](auto withA, const std::vector<TileBin> &side) -> int {
@@ -983,7 +993,7 @@ static int batch_run_tiles(const Env &e, glx_batch_instance *inst, int32_t n, in
     int host_err = 0;
     std::vector<int> sw(sweeps ? 2 * (size_t)n * nsteps : 0);
     st = hipMemcpyAsync(state.data(), d_state, sizeof(int) * 8 * n, hipMemcpyDeviceToHost, e.stream);
-    if (st == hipSuccess) st = hipMemcpyAsync(&host_err, e.err, sizeof(int), hipMemcpyDeviceToHost, e.stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(&host_err, ts.err, sizeof(int), hipMemcpyDeviceToHost, e.stream);
     if (st == hipSuccess && sweeps)
         st = hipMemcpyAsync(sw.data(), d_sw, sizeof(int) * sw.size(), hipMemcpyDeviceToHost, e.stream);
     if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
@@ -1075,6 +1085,17 @@ int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_
 
 // ---- batched CG -----------------------------------------------------------------
 
+// f(integral_constant NW) for the waves per instance of a batch of n: all
+// of a CU's for its share of the instances, four at least.
+template <typename R, typename F> static int with_batch_cg_waves(const Env &e, int32_t n, F &&f) {
+    constexpr int MOST = BatchCGWaves<R>::PER_CU;
+    const int each = MOST / std::max(1, (n + e.num_cus - 1) / e.num_cus);
+    if constexpr (MOST >= 16)
+        if (each >= 16) return f(std::integral_constant<int, 16>{});
+    if (each >= 8) return f(std::integral_constant<int, 8>{});
+    return f(std::integral_constant<int, 4>{});
+}
+
 template <typename R, int LL>
 static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, int32_t max_iters, double rtol,
                          int32_t per_launch, int32_t stall_iters, const double *init_state) {
@@ -1116,14 +1137,10 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
         for (int k = 0; k < 2; ++k) { c.dirA[k] = withA ? (R *)w : nullptr; if (withA) w += al(Nab * sizeof(R)); }
     }
     st = hipMemcpyAsync(d_inst, h.data(), sizeof(CGInst<R>) * n, hipMemcpyHostToDevice, e.stream);
-    if (st == hipSuccess) st = hipMemsetAsync(d_state, 0, s_state + off[n], e.stream);
+    if (st == hipSuccess) st = hipMemsetAsync(d_state, 0, s_state, e.stream);
     if (st == hipSuccess && init_state)
         st = hipMemcpyAsync(d_state, init_state, sizeof(double) * CG_NSTATE * n, hipMemcpyHostToDevice, e.stream);
     if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run upload");
-    int per_cu = 0;
-    st = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_cg<R, LL>, 256, 0);
-    if (st != hipSuccess) return check_hip(st, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-    const int grid = std::max(1, std::min(n, per_cu * e.num_cus));
     const int chunk = per_launch > 0 ? per_launch : 50;
     int it_min = max_iters;  // fewest iterations any instance starts with
     for (int i = 0; i < n; ++i) it_min = std::min(it_min, init_state ? (int)init_state[CG_NSTATE * i + CG_IT] : 0);
@@ -1133,9 +1150,18 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     st = hipEventRecord(e.kev0, e.stream);
     if (st != hipSuccess) return check_hip(st, "hipEventRecord");
     for (int done = it_min; done < max_iters; done += chunk) {
-        hipLaunchKernelGGL((k_batch_cg<R, LL>), dim3(grid), dim3(256), 0, e.stream, d_inst, d_state, n,
-                           std::min(chunk, max_iters - done), max_iters, rtol, stall_iters);
-        GLX_LAUNCH_CHECK("k_batch_cg");
+        const int rc = with_batch_cg_waves<R>(e, n, [&](auto nw) {
+            constexpr int NW = decltype(nw)::value;
+            int per_cu = 0;
+            const hipError_t so = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_cg<R, LL, NW>, NW * WAVE, 0);
+            if (so != hipSuccess) return check_hip(so, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+            const int grid = std::max(1, std::min(n, per_cu * e.num_cus));
+            hipLaunchKernelGGL((k_batch_cg<R, LL, NW>), dim3(grid), dim3(NW * WAVE), 0, e.stream, d_inst, d_state, n,
+                               std::min(chunk, max_iters - done), max_iters, rtol, stall_iters);
+            GLX_LAUNCH_CHECK("k_batch_cg");
+            return (int)GLX_OK;
+        });
+        if (rc) return rc;
         st = hipMemcpyAsync(hs.data(), d_state, sizeof(double) * CG_NSTATE * n, hipMemcpyDeviceToHost, e.stream);
         if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
         if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run readback");
