@@ -342,6 +342,12 @@ int glx_supercurrent_density(int prec, glx_grid g, const uint8_t *mt, const void
 int glx_bulk_observables(int prec, glx_grid g, double kappa2, double H, const uint8_t *mt,
                          const void *psi, const void *abei, const void *ab, void *B, void *J,
                          void *Js);
+/* The same results with B and the a and b parts of J and J_s each in column
+ * order (B[i * (Ny - 1) + j], and so on): what a host program that indexes
+ * [i, j] reads without a transposition. */
+int glx_bulk_observables_cols(int prec, glx_grid g, double kappa2, double H, const uint8_t *mt,
+                              const void *psi, const void *abei, const void *ab, void *B, void *J,
+                              void *Js);
 
 /* Total GL free energy, FP64 accumulation, returned on the host
  * (free_energy_pseudodensity, observables.h:250-362, + Reduction.gsum,

@@ -106,6 +106,7 @@ _PROTOS = {
     "glx_cg_energy_wait": [P_double],
     "glx_bulk_observables": [c_int, Grid, c_double, c_double, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                              c_void_p, c_void_p],
+    "glx_bulk_observables_cols": [c_int, Grid, c_double, c_double] + [c_void_p] * 7,
     "glx_sum": [c_int, c_void_p, c_i64, c_i32, P_double],
     "glx_sum_v": [c_int, c_void_p, c_i64, c_i32, c_i32, P_double],
     "glx_pr_sums": [c_int, c_void_p, c_void_p, c_i64, P_double],

@@ -454,7 +454,12 @@ int glx_supercurrent_density(int prec, glx_grid g, const uint8_t *mt, const void
 
 int glx_bulk_observables(int prec, glx_grid g, double kappa2, double H, const uint8_t *mt, const void *psi,
                          const void *abei, const void *ab, void *B, void *J, void *Js) {
-    GLX_DISPATCH(prec, bulk_observables(g_ctx.env, g, kappa2, H, mt, psi, abei, ab, B, J, Js));
+    GLX_DISPATCH(prec, bulk_observables(g_ctx.env, g, kappa2, H, mt, psi, abei, ab, B, J, Js, false));
+}
+
+int glx_bulk_observables_cols(int prec, glx_grid g, double kappa2, double H, const uint8_t *mt, const void *psi,
+                              const void *abei, const void *ab, void *B, void *J, void *Js) {
+    GLX_DISPATCH(prec, bulk_observables(g_ctx.env, g, kappa2, H, mt, psi, abei, ab, B, J, Js, true));
 }
 
 int glx_free_energy(int prec, glx_grid g, double kappa2, double eps, const void *eps_map, double H,

@@ -82,7 +82,7 @@ template <typename R> struct L {
     static int supercurrent_density(const Env &e, glx_grid g, const uint8_t *mt, const void *psi, const void *abei,
                                     const void *ab, void *Js);
     static int bulk_observables(const Env &e, glx_grid g, double kappa2, double H, const uint8_t *mt, const void *psi,
-                                const void *abei, const void *ab, void *B, void *J, void *Js);
+                                const void *abei, const void *ab, void *B, void *J, void *Js, bool cols);
     static int free_energy(const Env &e, glx_grid g, double kappa2, double eps, const void *eps_map, double H,
                            const uint8_t *mt, const void *psi, const void *abei, const void *ab, double *F);
     static int vortex_cells(const Env &e, glx_grid g, const void *psi, const void *ab, const void *abi, double H,

@@ -1343,10 +1343,17 @@ int L<R>::supercurrent_density(const Env &e, glx_grid g, const uint8_t *mt, cons
 
 template <typename R>
 int L<R>::bulk_observables(const Env &e, glx_grid g, double kappa2, double H, const uint8_t *mt, const void *psi,
-                           const void *abei, const void *ab, void *B, void *J, void *Js) {
+                           const void *abei, const void *ab, void *B, void *J, void *Js, bool cols) {
     if (!grid_ok(g) || (Js && !psi)) return set_error(GLX_E_ARG, "glx_bulk_observables: invalid arguments");
     if (!B && !J && !Js) return GLX_OK;
     const Geo G = make_geo(g.Nx, g.Ny, g.dx, g.dy);
+    if (cols) {
+        const long nt = (long)((g.Nx + OBS_TILE - 1) / OBS_TILE) * ((g.Ny + OBS_TILE - 1) / OBS_TILE);
+        hipLaunchKernelGGL(k_bulk_observables_cols<R>, dim3(grid_blocks(nt, 1)), dim3(256), 0, e.stream, G, R(kappa2),
+                           R(H), mt, (const cplx<R> *)psi, (const R *)abei, (const R *)ab, (R *)B, (R *)J, (R *)Js);
+        GLX_LAUNCH_CHECK("k_bulk_observables_cols");
+        return GLX_OK;
+    }
     hipLaunchKernelGGL(k_bulk_observables<R>, dim3(grid_blocks(G.N)), dim3(256), 0, e.stream, G, R(kappa2), R(H), mt,
                        (const cplx<R> *)psi, (const R *)abei, (const R *)ab, (R *)B, (R *)J, (R *)Js);
     GLX_LAUNCH_CHECK("k_bulk_observables");

@@ -38,27 +38,37 @@ class Observables:
         """B per cell from abei + ab (observables.py:36-58)."""
         self._sync_device()
         out = self.vars._tmp_cell_var_h()
-        nat.call("glx_magnetic_field", self.par.prec, self._grid(),
-                 nat.ptr(self.params.external_irregular_vector_potential_h()),
-                 nat.ptr(self.vars.vector_potential_h()), out.ptr)
-        c = self.cfg
-        return np.reshape(out.get(), (c.Nyc, c.Nxc)).T.copy()
+        self._cols(out, None, None)
+        return self._cells(out)
+
+    def _cols(self, B, J, Js):
+        """B, J and J_s of the state into device arrays (None: not), each
+        in column order: [i, j] of the host arrays."""
+        p = self.params
+        nat.call("glx_bulk_observables_cols", self.par.prec, self._grid(),
+                 float(p.gl_parameter_squared_h()) if p.solveA else 0.0, float(p.homogeneous_external_field),
+                 nat.ptr(self.mesh.material_tiling_h()), self.vars.order_parameter_h().ptr,
+                 nat.ptr(p.external_irregular_vector_potential_h()), nat.ptr(self.vars.vector_potential_h()),
+                 nat.ptr(B), nat.ptr(J), nat.ptr(Js))
+
+    def _host(self, dev, first, shape):
+        out = np.empty(shape, dtype=dev.dtype)
+        nat.call("glx_memcpy_d2h", out.ctypes.data, dev.ptr + int(first) * dev.dtype.itemsize, out.nbytes)
+        return out
+
+    def _cells(self, dev):
+        return self._host(dev, 0, (int(self.cfg.Nxc), int(self.cfg.Nyc)))
 
     def _edge_pair(self, dev):
         c = self.cfg
-        v = dev.get()
-        a = np.reshape(v[:c.Na], (c.Nya, c.Nxa)).T.copy()
-        b = np.reshape(v[c.Na:], (c.Nyb, c.Nxb)).T.copy()
-        return a, b
+        return self._host(dev, 0, (int(c.Nxa), int(c.Nya))), self._host(dev, c.Na, (int(c.Nxb), int(c.Nyb)))
 
     @property
     def supercurrent_density(self):
         """J_s on links (observables.py:61-83)."""
         self._sync_device()
         out = self.vars._tmp_edge_var_h()
-        nat.call("glx_supercurrent_density", self.par.prec, self._grid(), nat.ptr(self.mesh.material_tiling_h()),
-                 self.vars.order_parameter_h().ptr, nat.ptr(self.params.external_irregular_vector_potential_h()),
-                 nat.ptr(self.vars.vector_potential_h()), out.ptr)
+        self._cols(None, None, out)
         return self._edge_pair(out)
 
     @property
@@ -69,16 +79,13 @@ class Observables:
             return self.supercurrent_density
         self._sync_device()
         out = self.vars._tmp_edge_var_h()
-        nat.call("glx_current_density", self.par.prec, self._grid(), float(self.params.gl_parameter_squared_h()),
-                 float(self.params.homogeneous_external_field),
-                 nat.ptr(self.params.external_irregular_vector_potential_h()),
-                 nat.ptr(self.vars.vector_potential_h()), out.ptr)
+        self._cols(None, out, None)
         return self._edge_pair(out)
 
     @property
     def normalcurrent_density(self):
         """J - J_s on links (observables.py:113-121); with A solved, J and
-        J_s come from one fused pass (glx_bulk_observables)."""
+        J_s come from one fused pass (glx_bulk_observables_cols)."""
         if not self.params.solveA:
             jx, jy = self.current_density
             jsx, jsy = self.supercurrent_density
@@ -100,12 +107,8 @@ class Observables:
         B = self.vars._tmp_cell_var_h() if want_B else None
         J = self.vars._tmp_edge_var_h() if p.solveA else None
         Js = self._edge2
-        nat.call("glx_bulk_observables", self.par.prec, self._grid(),
-                 float(p.gl_parameter_squared_h()) if p.solveA else 0.0, float(p.homogeneous_external_field),
-                 nat.ptr(self.mesh.material_tiling_h()), self.vars.order_parameter_h().ptr,
-                 nat.ptr(p.external_irregular_vector_potential_h()), nat.ptr(self.vars.vector_potential_h()),
-                 nat.ptr(B), nat.ptr(J), Js.ptr)
-        Bh = np.reshape(B.get(), (c.Nyc, c.Nxc)).T.copy() if want_B else None
+        self._cols(B, J, Js)
+        Bh = self._cells(B) if want_B else None
         js = self._edge_pair(Js)
         # J = J_s when kappa = inf (observables.py:86-110)
         jj = self._edge_pair(J) if J is not None else (js[0].copy(), js[1].copy())
