@@ -60,16 +60,22 @@ __device__ __forceinline__ void block_sums(const double (&acc)[L], double (&part
     __syncthreads();
 }
 
-// The threads of an instance's workgroup: as many as fill the registers of
-// the CUs with the batch's instances resident together. A wave waits out the
-// memory latency of its nodes' loads, so an instance alone on a CU with the
-// four waves of a full batch leaves the CU idle most of the time: 256
-// instances of 129 x 129 (FP32, kappa < inf), per iteration: 718 us with 4
-// waves, 420 with 8, 306 with 16, of which 42 move the update at the rate of
-// the memory. FP32 stays below 128 VGPRs (16 waves a CU; 1024
-// instances are resident at 4 waves each), FP64 below 256 (8 waves).
-template <typename R> struct BatchCGWaves { static constexpr int PER_CU = 8; };
-template <> struct BatchCGWaves<float> { static constexpr int PER_CU = 16; };
+// The waves of an instance's workgroup and the workgroups that share a CU.
+// FP32: 16 waves for instances of more than BATCH_CG_SMALL nodes, 4 for the
+// others, both at 128 VGPRs, so 16 waves a CU. A wave waits out the memory
+// latency of its nodes' loads: with one instance a CU, 4 waves leave it idle
+// most of the time, and with four or more, one instance at a time with all
+// waves on it is no slower. Small instances wait for the sums and the line
+// search, which several a CU overlap. Kernel time of 8 iterations, kappa <
+// inf, 4 / 16 waves: 256 instances of 129 x 129 5.75 / 2.44 ms, 1024 of them
+// 10.3 / 9.5; 256 and 1024 of 65 x 65 1.36 / 0.69 and 2.63 / 2.59, of 49 x 49
+// 0.83 / 0.49 and 1.23 / 1.82. An instance's form depends on its own size
+// only: it ends in the same bits in any batch. FP64 keeps 4 waves and the
+// order of its sums: the line search resolves a step to 1e-8 only, and another
+// order would move an FP64 path by as much.
+constexpr long BATCH_CG_SMALL = 4096;
+template <typename R> struct BatchCGWaves { static constexpr int MOST = 4, PER_CU = 4; };
+template <> struct BatchCGWaves<float> { static constexpr int MOST = 16, PER_CU = 16; };
 
 // Stall rule (stall_iters > 0): an instance whose relative gradient norm
 // has not halved within stall_iters iterations stops with flag 2 (the

@@ -1085,15 +1085,18 @@ int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_
 
 // ---- batched CG -----------------------------------------------------------------
 
-// f(integral_constant NW) for the waves per instance of a batch of n: all
-// of a CU's for its share of the instances, four at least.
-template <typename R, typename F> static int with_batch_cg_waves(const Env &e, int32_t n, F &&f) {
-    constexpr int MOST = BatchCGWaves<R>::PER_CU;
-    const int each = MOST / std::max(1, (n + e.num_cus - 1) / e.num_cus);
-    if constexpr (MOST >= 16)
-        if (each >= 16) return f(std::integral_constant<int, 16>{});
-    if (each >= 8) return f(std::integral_constant<int, 8>{});
-    return f(std::integral_constant<int, 4>{});
+// `iters` iterations of n instances with NW waves each.
+template <typename R, int LL, int NW>
+static int batch_cg_launch(const Env &e, const CGInst<R> *d_inst, double *d_state, int n, int iters, int max_iters,
+                           double rtol, int stall_iters) {
+    int per_cu = 0;
+    const hipError_t st = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_cg<R, LL, NW>, NW * WAVE, 0);
+    if (st != hipSuccess) return check_hip(st, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+    const int grid = std::max(1, std::min(n, per_cu * e.num_cus));
+    hipLaunchKernelGGL((k_batch_cg<R, LL, NW>), dim3(grid), dim3(NW * WAVE), 0, e.stream, d_inst, d_state, n, iters,
+                       max_iters, rtol, stall_iters);
+    GLX_LAUNCH_CHECK("k_batch_cg");
+    return GLX_OK;
 }
 
 template <typename R, int LL>
@@ -1116,12 +1119,21 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     CGInst<R> *d_inst = (CGInst<R> *)blk;
     double *d_state = (double *)(blk + s_inst);
     char *work = blk + s_inst + s_state;
+    // the ns small instances first, each at place at[i]
+    std::vector<int> at(n);
+    int ns = 0, place = 0;
+    auto small = [&](int i) { return (long)inst[i].g.Nx * inst[i].g.Ny <= BATCH_CG_SMALL; };
+    for (int i = 0; i < n; ++i)
+        if (small(i)) at[i] = ns++;
+    place = ns;
+    for (int i = 0; i < n; ++i)
+        if (!small(i)) at[i] = place++;
     std::vector<CGInst<R>> h(n);
     for (int i = 0; i < n; ++i) {
         const glx_batch_cg_instance &I = inst[i];
         const glx_grid &g = I.g;
         const size_t N = (size_t)g.Nx * g.Ny, Nab = (size_t)(g.Nx - 1) * g.Ny + (size_t)g.Nx * (g.Ny - 1);
-        CGInst<R> &c = h[i];
+        CGInst<R> &c = h[at[i]];
         c.g = make_geo(g.Nx, g.Ny, g.dx, g.dy);
         c.kappa2 = R(I.kappa2);
         c.eps = R(I.eps);
@@ -1138,29 +1150,26 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     }
     st = hipMemcpyAsync(d_inst, h.data(), sizeof(CGInst<R>) * n, hipMemcpyHostToDevice, e.stream);
     if (st == hipSuccess) st = hipMemsetAsync(d_state, 0, s_state, e.stream);
+    std::vector<double> hs(CG_NSTATE * (size_t)n, 0.0);
+    if (init_state)
+        for (int i = 0; i < n; ++i)
+            std::copy(init_state + CG_NSTATE * (size_t)i, init_state + CG_NSTATE * (size_t)(i + 1),
+                      hs.begin() + CG_NSTATE * (size_t)at[i]);
     if (st == hipSuccess && init_state)
-        st = hipMemcpyAsync(d_state, init_state, sizeof(double) * CG_NSTATE * n, hipMemcpyHostToDevice, e.stream);
+        st = hipMemcpyAsync(d_state, hs.data(), sizeof(double) * CG_NSTATE * n, hipMemcpyHostToDevice, e.stream);
     if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run upload");
     const int chunk = per_launch > 0 ? per_launch : 50;
     int it_min = max_iters;  // fewest iterations any instance starts with
     for (int i = 0; i < n; ++i) it_min = std::min(it_min, init_state ? (int)init_state[CG_NSTATE * i + CG_IT] : 0);
-    std::vector<double> hs(CG_NSTATE * (size_t)n);
-    if (init_state) std::copy(init_state, init_state + CG_NSTATE * (size_t)n, hs.begin());
-    else std::fill(hs.begin(), hs.end(), 0.0);
     st = hipEventRecord(e.kev0, e.stream);
     if (st != hipSuccess) return check_hip(st, "hipEventRecord");
     for (int done = it_min; done < max_iters; done += chunk) {
-        const int rc = with_batch_cg_waves<R>(e, n, [&](auto nw) {
-            constexpr int NW = decltype(nw)::value;
-            int per_cu = 0;
-            const hipError_t so = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_cg<R, LL, NW>, NW * WAVE, 0);
-            if (so != hipSuccess) return check_hip(so, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-            const int grid = std::max(1, std::min(n, per_cu * e.num_cus));
-            hipLaunchKernelGGL((k_batch_cg<R, LL, NW>), dim3(grid), dim3(NW * WAVE), 0, e.stream, d_inst, d_state, n,
-                               std::min(chunk, max_iters - done), max_iters, rtol, stall_iters);
-            GLX_LAUNCH_CHECK("k_batch_cg");
-            return (int)GLX_OK;
-        });
+        const int iters = std::min(chunk, max_iters - done);
+        int rc = GLX_OK;
+        if (ns > 0) rc = batch_cg_launch<R, LL, 4>(e, d_inst, d_state, ns, iters, max_iters, rtol, stall_iters);
+        if (!rc && ns < n)
+            rc = batch_cg_launch<R, LL, BatchCGWaves<R>::MOST>(e, d_inst + ns, d_state + CG_NSTATE * ns, n - ns, iters,
+                                                              max_iters, rtol, stall_iters);
         if (rc) return rc;
         st = hipMemcpyAsync(hs.data(), d_state, sizeof(double) * CG_NSTATE * n, hipMemcpyDeviceToHost, e.stream);
         if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
@@ -1176,7 +1185,7 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     float kms = 0.f;
     if (hipEventElapsedTime(&kms, e.kev0, e.kev1) == hipSuccess && e.last_kernel_ms) *e.last_kernel_ms = kms;
     for (int i = 0; i < n; ++i) {
-        const double *sv = hs.data() + CG_NSTATE * i;
+        const double *sv = hs.data() + CG_NSTATE * (size_t)at[i];
         inst[i].iters = (int32_t)sv[CG_IT];
         inst[i].converged = sv[CG_DONE] == 1.0 ? 1 : 0;
         inst[i].stalled = sv[CG_DONE] == 2.0 ? 1 : 0;

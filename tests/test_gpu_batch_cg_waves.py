@@ -1,7 +1,8 @@
-"""The batched CG gives an instance more waves the fewer instances share a
-CU. In batches that take each form: FP64, the first iteration of an instance
-among many is the oracle's steepest descent to the line minimum; FP32-mixed,
-an instance among many ends at the FP64 form's free energy."""
+"""The FP32-mixed batched CG gives instances of more than 4096 nodes sixteen
+waves and the others four; FP64 four. In batches that mix them: FP64, the
+first iteration of an instance among many is the oracle's steepest descent to
+the line minimum; FP32-mixed, an instance among many ends at the FP64 form's
+free energy, and in the bits it ends in alone."""
 import numpy as np
 import pytest
 
@@ -26,7 +27,7 @@ def batch(n, dtype, init):
     return [make(0, 65, 40, 5.0, 0.3, dtype, init)] + filler + [make(1, 33, 29, 5.0, 0.1, dtype, init)]
 
 
-# one and two instances a CU of 256
+# fewer and more instances than 256 CUs
 @pytest.mark.parametrize("n", [3, 300])
 def test_first_iteration_is_line_minimum(n):
     from svirl_amd.batch import BatchCG
@@ -53,13 +54,23 @@ def test_first_iteration_is_line_minimum(n):
                 assert fa <= f(sx * ap, sy * aA) + 1e-12 * abs(fa)
 
 
-# one, two, three and five instances a CU of 256
-@pytest.mark.parametrize("n", [3, 300, 600, 1100])
+# 2600 and 957 nodes (four waves) beside 4355 (sixteen), and fewer or more
+# instances than the 256 CUs hold at once
+@pytest.mark.parametrize("n", [3, 300, 1100])
 def test_fp32_mixed_reaches_fp64_energy(n):
     from svirl_amd.batch import BatchCG
-    s64, s32 = batch(3, np.float64, 1.0), batch(n, np.float32, 1.0)
+
+    def sims(n, dtype):
+        b = batch(n, dtype, 1.0)
+        return b[:1] + [make(2, 65, 67, 5.0, 0.2, dtype, 1.0)] + b[1:]
+
+    s64, s32 = sims(3, np.float64), sims(n, np.float32)
+    alone = sims(3, np.float32)
     BatchCG(s64).cg(max_iter=3000, rtol=1e-6)
-    BatchCG(s32).cg(max_iter=3000, rtol=1e-4)
-    for a, b in ((s32[0], s64[0]), (s32[-1], s64[-1])):
+    iters, _, _ = BatchCG(s32).cg(max_iter=3000, rtol=1e-4)
+    for k, a, b in ((0, s32[0], s64[0]), (1, s32[1], s64[1]), (-1, s32[-1], s64[-1])):
         fa, fb = a.observables.free_energy_fp64(), b.observables.free_energy_fp64()
         assert abs(fa - fb) <= 1e-5 * abs(fb)
+        it1, _, _ = BatchCG([alone[k]]).cg(max_iter=3000, rtol=1e-4)
+        assert it1[0] == iters[k]
+        assert np.array_equal(alone[k].vars.order_parameter, a.vars.order_parameter)
