@@ -20,13 +20,24 @@
 
 namespace glx {
 
-// Waves of a row-marching CG pass: about 16 rows per wave, at most 4096
-// waves (1024 workgroups, the partials' capacity). The passes hand out the
+// Waves of a row-marching CG pass: 16 rows per wave, FP32 at least two waves
+// a SIMD (2048) where there are rows for them, at most 4096 waves (1024
+// workgroups, the partials' capacity). On small grids a pass lasts as long as
+// a wave's rows, one after the other; the rows above and below that every
+// wave reads besides its own cost nothing while the chip is not full. Per
+// iteration of the FP32-mixed CG, kappa < inf, with 16 rows / one / this rule:
+// 129^2 87 / 48 / 48 us, 385^2 89 / 54 / 54, 1025^2 108 / 100 / 86 (more waves
+// leave more partial sums to reduce), 2049^2 228 with any. FP64 keeps 16 rows,
+// and with them the order of its sums: its line search, on the host by the
+// reference's minimiser, resolves a step to 1e-8, and any other order moves
+// the path by as much; it also takes three times as long as the passes. The
+// passes hand out the
 // rows row-major (for_rows_rm): waves of consecutive index march the same
 // rows of adjacent strips, so the chip reads whole grid rows together.
-inline long cg_row_waves(int Nx, int Ny) {
+template <typename R> inline long cg_row_waves(int Nx, int Ny) {
     const long T = (long)nstrips_of<1>(Nx) * Ny;
     long W = (T + 15) / 16;
+    if (std::is_same<R, float>::value && W < 2048) W = T < 2048 ? T : 2048;
     if (W > 4 * RED_MAX_BLOCKS) W = 4 * RED_MAX_BLOCKS;
     return W < 1 ? 1 : W;
 }

@@ -1561,7 +1561,7 @@ static int gradient_pass_launch(const Env &e, glx_grid g, double kappa2, double 
     // iteration takes 0.70 ms this way against 0.72 ms with three (its
     // traffic per node barely changes, so the gain is in how the passes
     // overlap their loads, not in bytes)
-    const long W = fit_row_waves(fn, cg_row_waves(g.Nx, g.Ny), e.num_cus, 2);
+    const long W = fit_row_waves(fn, cg_row_waves<R>(g.Nx, g.Ny), e.num_cus, 2);
     const int nb = (int)((W + 3) / 4);
     *nb_out = nb;
     const R k2 = R(kappa2), ep = R(eps), h = R(H);
@@ -1711,7 +1711,7 @@ int L<R>::cg_direction_step(const Env &e, glx_grid g, double kappa2, double eps,
     if (kappa2 > 0.0 && !(abei || ab)) return set_error(GLX_E_ARG, "glx_cg_direction_step: finite kappa needs ab");
     const Geo G = make_geo(g.Nx, g.Ny, g.dx, g.dy);
     const long W = fit_row_waves(withA ? (const void *)k_coef_dir_rows<R, 17> : (const void *)k_coef_dir_rows<R, 5>,
-                                 cg_row_waves(g.Nx, g.Ny), e.num_cus);
+                                 cg_row_waves<R>(g.Nx, g.Ny), e.num_cus);
     const int nb = (int)((W + 3) / 4);
     const double dxdy = double(R(g.dx)) * double(R(g.dy));
     DirUpdate<R> U{(const cplx<R> *)dpsi, (const cplx<R> *)jac, (const R *)dab, (const R *)jacA,
