@@ -188,13 +188,31 @@ __device__ __forceinline__ R psi_den(const PsiSweepArgs<R> &A, const cplx<R> &rh
     }
 }
 
+// n / den from r = 1 / den rounded: q = n r, then q + r (n - q den) with one
+// fma each, which is the IEEE quotient but for cases a 2^-52 part of inputs
+// can reach (v_div_fixup covers zeros, infinities and NaN), in 4 instructions
+// against about 11. The FP64 passes issue VALU instructions 70% of the time;
+// with one reciprocal a node and pass for the six quotients of three sweeps,
+// and none for A's constant denominators, a step on 4097 x 4097 takes 3.90 ms
+// where it took 4.03 (the two registers come from shifting the left link's
+// factors anew in each stage of psi_rows3).
+__device__ __forceinline__ double div_by(double n, double den, double r) {
+    const double q = n * r;
+    const double e = __builtin_fma(-q, den, n);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(e, r, q), den, n);
+}
+
+// 1 / den for psi_apply (FP64).
+__device__ __forceinline__ double psi_rden(double den) { return 1.0 / den; }
+__device__ __forceinline__ float psi_rden(float den) { return den; }
+
 // psi_apply: the off-diagonal part and the division, from the neighbours pl,
 // pr, pm, pp (left, right, down, up) and the link factors (c, s) = (cos, sin)
 // of dx a_left, dx a, dy b_down, dy b. A link that touches no material cell
 // carries the factors (0, 0) (mask_link), which makes its term 0 as the
 // reference's link weight 0 does.
 template <typename R>
-__device__ __forceinline__ cplx<R> psi_apply(const PsiSweepArgs<R> &A, const cplx<R> &rhs, R den, R pl_re, R pl_im,
+__device__ __forceinline__ cplx<R> psi_apply(const PsiSweepArgs<R> &A, const cplx<R> &rhs, R den, R rden, R pl_re, R pl_im,
                                              R pr_re, R pr_im, const cplx<R> &pm, const cplx<R> &pp, R cal, R sal,
                                              R ca, R sa, R cbm, R sbm, R cb, R sb) {
     // U(-dx a_left) psi_left, U(dx a) psi_right, U(-dy b_down) psi_down, U(dy b) psi_up
@@ -205,7 +223,7 @@ __device__ __forceinline__ cplx<R> psi_apply(const PsiSweepArgs<R> &A, const cpl
     const R nre = rhs.re + A.dt * (A.idx2 * (m0r + p0r) + A.idy2 * (q0mr + q0pr));
     const R nim = rhs.im + A.dt * (A.idx2 * (m0i + p0i) + A.idy2 * (q0mi + q0pi));
     if constexpr (std::is_same<R, float>::value) return {nre * den, nim * den};
-    else return {nre / den, nim / den};
+    else return {div_by(nre, den, rden), div_by(nim, den, rden)};
 }
 
 // psi_apply for FP32 passes with two products folded in per row: the link
@@ -298,8 +316,9 @@ __device__ __forceinline__ R psi_rows(const PsiSweepArgs<R> &A, int s, int ja, i
             cplx<R> nxt = {R(0), R(0)};
             if (inside) {
                 if (noisy && A.jstep == 0 && A.langevin_c > R(1.0e-32)) psi_noise(A, (uint32_t)(c + rowoff), rhs);
-                nxt = psi_apply(A, rhs, psi_den(A, rhs, e, mm, mp, pmc, ppc), pl_re, pl_im, pr_re, pr_im, pm, pp, cal,
-                                sal, ca, sa, cbm, sbm, cb, sb);
+                const R den = psi_den(A, rhs, e, mm, mp, pmc, ppc);
+                nxt = psi_apply(A, rhs, den, psi_rden(den), pl_re, pl_im, pr_re, pr_im, pm, pp, cal, sal, ca, sa, cbm,
+                                sbm, cb, sb);
             }
             if (noisy && A.jstep == 0) st(A.rhs_out, c + rowoff, rhs);
             st_at(A.psi_next + rowoff, 2 * X.cc * (uint32_t)sizeof(R), nxt);
@@ -374,7 +393,7 @@ __device__ __forceinline__ void psi_rows2(const PsiSweepArgs<R> &A, int s, int j
     // second sweep window (row u = t - 1): psi^{j+1} at u-1, u; U of a(u),
     // b(u-1); rhs, diagonal and material test of node (c, u)
     cplx<R> qm = zero, qc = zero, rhs_u = zero;
-    R ca2 = R(0), sa2 = R(0), cal2 = R(0), sal2 = R(0), cb2 = R(0), sb2 = R(0), den_u = R(1);
+    R ca2 = R(0), sa2 = R(0), cal2 = R(0), sal2 = R(0), cb2 = R(0), sb2 = R(0), den_u = R(1), rden_u = R(1);
     bool in_u = false;
 
     auto row = [&](const PsiRow<R> &cu, int t) {
@@ -399,14 +418,15 @@ __device__ __forceinline__ void psi_rows2(const PsiSweepArgs<R> &A, int s, int j
 
         // first sweep at row t -> psi^{j+1}(t)
         cplx<R> q = zero;
-        R den = R(1);
+        R den = R(1), rden = R(1);
         {
             const R pl_re = shfl_up1(pc.re), pl_im = shfl_up1(pc.im);
             const R pr_re = shfl_dn1(pc.re), pr_im = shfl_dn1(pc.im);
             if (mid && real && inside) {
                 if (noise_on) psi_noise(A, (uint32_t)(c + rowoff), rhs);
                 den = psi_den(A, rhs, e, mm, mp, pmc, ppc);
-                q = psi_apply(A, rhs, den, pl_re, pl_im, pr_re, pr_im, pm, pp, cal, sal, ca, sa, cb1, sb1, cb, sb);
+                rden = psi_rden(den);
+                q = psi_apply(A, rhs, den, rden, pl_re, pl_im, pr_re, pr_im, pm, pp, cal, sal, ca, sa, cb1, sb1, cb, sb);
             }
             if (own && real && t >= ja && t < jb) {
                 if (noisy && A.jstep == 0) st(A.rhs_out, c + rowoff, rhs);
@@ -421,7 +441,7 @@ __device__ __forceinline__ void psi_rows2(const PsiSweepArgs<R> &A, int s, int j
             if (own) {
                 cplx<R> nxt = zero;
                 if (in_u)
-                    nxt = psi_apply(A, rhs_u, den_u, pl_re, pl_im, pr_re, pr_im, qm, q, cal2, sal2, ca2, sa2, cb2, sb2,
+                    nxt = psi_apply(A, rhs_u, den_u, rden_u, pl_re, pl_im, pr_re, pr_im, qm, q, cal2, sal2, ca2, sa2, cb2, sb2,
                                     cb1, sb1);
                 st_at(A.psi_next + (size_t)Nx * u, 2 * X.cc * (uint32_t)sizeof(R), nxt);
                 r2 = fmax(r2, fmax(fabs(nxt.re - qc.re), fabs(nxt.im - qc.im)));
@@ -438,6 +458,7 @@ __device__ __forceinline__ void psi_rows2(const PsiSweepArgs<R> &A, int s, int j
         sal2 = sal;
         in_u = inside;
         den_u = den;
+        rden_u = rden;
         rhs_u = rhs;
         pm = pc;
         pc = pp;
@@ -508,12 +529,12 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
     // sweep j+1 window (row u = t - 1): psi^{j+1} at u-1, u; U of a(u),
     // b(u-1); rhs, diagonal and material test of node (c, u)
     cplx<R> qm = zero, qc = zero, rhs_u = zero;
-    R ca2 = R(0), sa2 = R(0), cal2 = R(0), sal2 = R(0), cb2 = R(0), sb2 = R(0), den_u = R(1);
+    R ca2 = R(0), sa2 = R(0), cb2 = R(0), sb2 = R(0), den_u = R(1), rden_u = R(1);
     bool in_u = false;
     // sweep j+2 window (row v = t - 2): psi^{j+2} at v-1, v; U of a(v),
     // b(v-1); rhs, diagonal and material test of node (c, v)
     cplx<R> wm = zero, wc = zero, rhs_v = zero;
-    R ca3 = R(0), sa3 = R(0), cal3 = R(0), sal3 = R(0), cb3 = R(0), sb3 = R(0), den_v = R(1);
+    R ca3 = R(0), sa3 = R(0), cb3 = R(0), sb3 = R(0), den_v = R(1), rden_v = R(1);
     bool in_v = false;
 
     auto row = [&](const PsiRow<R> &cu, int t) {
@@ -538,14 +559,15 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
 
         // sweep j at row t -> psi^{j+1}(t)
         cplx<R> q = zero;
-        R den = R(1);
+        R den = R(1), rden = R(1);
         {
             const R pl_re = shfl_up1(pc.re), pl_im = shfl_up1(pc.im);
             const R pr_re = shfl_dn1(pc.re), pr_im = shfl_dn1(pc.im);
             if (mid1 && real && inside) {
                 if (noise_on) psi_noise(A, (uint32_t)(c + rowoff), rhs);
                 den = psi_den(A, rhs, e, mm, mp, pmc, ppc);
-                q = psi_apply(A, rhs, den, pl_re, pl_im, pr_re, pr_im, pm, pp, cal, sal, ca, sa, cb1, sb1, cb, sb);
+                rden = psi_rden(den);
+                q = psi_apply(A, rhs, den, rden, pl_re, pl_im, pr_re, pr_im, pm, pp, cal, sal, ca, sa, cb1, sb1, cb, sb);
             }
             if (own && real && t >= ja && t < jb) {
                 if (noisy && A.jstep == 0) st(A.rhs_out, c + rowoff, rhs);
@@ -558,8 +580,9 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
         if (u >= 0 && u < Ny) {
             const R pl_re = shfl_up1(qc.re), pl_im = shfl_up1(qc.im);
             const R pr_re = shfl_dn1(qc.re), pr_im = shfl_dn1(qc.im);
+            const R cal2 = shfl_up1(ca2), sal2 = shfl_up1(sa2);
             if (mid2 && in_u)
-                w = psi_apply(A, rhs_u, den_u, pl_re, pl_im, pr_re, pr_im, qm, q, cal2, sal2, ca2, sa2, cb2, sb2, cb1,
+                w = psi_apply(A, rhs_u, den_u, rden_u, pl_re, pl_im, pr_re, pr_im, qm, q, cal2, sal2, ca2, sa2, cb2, sb2, cb1,
                               sb1);
             if (own && u >= ja && u < jb) r2 = fmax(r2, fmax(fabs(w.re - qc.re), fabs(w.im - qc.im)));
         }
@@ -568,10 +591,11 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
         if (v >= ja) {
             const R pl_re = shfl_up1(wc.re), pl_im = shfl_up1(wc.im);
             const R pr_re = shfl_dn1(wc.re), pr_im = shfl_dn1(wc.im);
+            const R cal3 = shfl_up1(ca3), sal3 = shfl_up1(sa3);
             if (own) {
                 cplx<R> nxt = zero;
                 if (in_v)
-                    nxt = psi_apply(A, rhs_v, den_v, pl_re, pl_im, pr_re, pr_im, wm, w, cal3, sal3, ca3, sa3, cb3, sb3,
+                    nxt = psi_apply(A, rhs_v, den_v, rden_v, pl_re, pl_im, pr_re, pr_im, wm, w, cal3, sal3, ca3, sa3, cb3, sb3,
                                     cb2, sb2);
                 st_at(A.psi_next + (size_t)Nx * v, 2 * X.cc * (uint32_t)sizeof(R), nxt);
                 r3 = fmax(r3, fmax(fabs(nxt.re - wc.re), fabs(nxt.im - wc.im)));
@@ -584,10 +608,9 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
         sb3 = sb2;
         ca3 = ca2;
         sa3 = sa2;
-        cal3 = cal2;
-        sal3 = sal2;
         in_v = in_u;
         den_v = den_u;
+        rden_v = rden_u;
         rhs_v = rhs_u;
         qm = qc;
         qc = q;
@@ -595,10 +618,9 @@ __device__ __forceinline__ void psi_rows3(const PsiSweepArgs<R> &A, int s, int j
         sb2 = sb1;
         ca2 = ca;
         sa2 = sa;
-        cal2 = cal;
-        sal2 = sal;
         in_u = inside;
         den_u = den;
+        rden_u = rden;
         rhs_u = rhs;
         pm = pc;
         pc = pp;
@@ -798,7 +820,7 @@ __device__ __forceinline__ void psi_rowsK(const PsiSweepArgs<R> &A, int s_, int 
                                       pp, cal, sal, ca, sa, cb1, sb1, cb, sb);
             } else {
                 rd = own_copy(rhs);
-                qa = psi_apply(A, rhs, d, shfl_up1(pc.re), shfl_up1(pc.im), shfl_dn1(pc.re), shfl_dn1(pc.im), pm, pp,
+                qa = psi_apply(A, rhs, d, psi_rden(d), shfl_up1(pc.re), shfl_up1(pc.im), shfl_dn1(pc.re), shfl_dn1(pc.im), pm, pp,
                                cal, sal, ca, sa, cb1, sb1, cb, sb);
             }
             const cplx<R> q = act ? qa : zero;
@@ -826,7 +848,7 @@ __device__ __forceinline__ void psi_rowsK(const PsiSweepArgs<R> &A, int s_, int 
                 wa = psi_apply_folded(W.rhs, W.den, shfl_up1(wc.re), shfl_up1(wc.im), shfl_dn1(wc.re), shfl_dn1(wc.im),
                                       wm, out[st_ - 1], W.cal, W.sal, W.ca, W.sa, W.cbd, W.sbd, ucb, usb);
             else
-                wa = psi_apply(A, W.rhs, W.den, shfl_up1(wc.re), shfl_up1(wc.im), shfl_dn1(wc.re), shfl_dn1(wc.im),
+                wa = psi_apply(A, W.rhs, W.den, psi_rden(W.den), shfl_up1(wc.re), shfl_up1(wc.im), shfl_dn1(wc.re), shfl_dn1(wc.im),
                                wm, out[st_ - 1], W.cal, W.sal, W.ca, W.sa, W.cbd, W.sbd, ucb, usb);
             const bool res = own && rs >= ja && rs < jb;  // rows of [ja, jb) lie in [0, Ny)
             cplx<R> w;
@@ -960,7 +982,7 @@ __device__ __forceinline__ R a_link_update(const ASweepArgs<R> &A, int j, R ra, 
     if (j + 1 < Ny) t2 = A.idy2 * ap + A.idxy * bc - A.idxy * brc;
     const R num = ra + A.dt_rho * (jl + rh) + A.dt_rho_kappa2 * dd * (t1 + t2);
     if constexpr (std::is_same<R, float>::value) return num * A.iden_a;
-    else return num / A.den_a;
+    else return div_by(num, A.den_a, A.iden_a);
 }
 
 // The b link (c, j) (td.h:412-456): blc = b(c-1, j), alc = a(c-1, j),
@@ -977,7 +999,7 @@ __device__ __forceinline__ R b_link_update(const ASweepArgs<R> &A, int c, R rb, 
     if (c + 1 < Nx) t2 = A.idx2 * brc + A.idxy * ac - A.idxy * ap;
     const R num = rb + A.dt_rho * (jl + rh) + A.dt_rho_kappa2 * dd * (t1 + t2);
     if constexpr (std::is_same<R, float>::value) return num * A.iden_b;
-    else return num / A.den_b;
+    else return div_by(num, A.den_b, A.iden_b);
 }
 
 // Supercurrent of a link, id * Im(conj psi0 U psi1) in the reference's form.

@@ -14,11 +14,7 @@
 // the whole solve, and one launch runs all steps of a run.
 //
 // The FP64 arithmetic is that of the row-marching passes (psi_rows, a_rows):
-// results and every sweep count equal theirs to the bit. The quotient
-// n / den is formed from the rounded reciprocal r of den (once per step):
-// q = n r, then q + r (n - q den) with one fma each, which is the IEEE
-// quotient but for cases a 2^-52 part of inputs can reach (v_div_fixup
-// covers zeros, infinities and NaN), in 4 instructions against about 12.
+// results and every sweep count equal theirs to the bit.
 //
 // FP32 psi solves carry the change d of a sweep and the sum D of the changes
 // instead of psi and its right-hand side: the solve is linear in psi, so
@@ -219,13 +215,6 @@ template <> struct TileSinCos<double> {
     }
 };
 
-// n / den from r = 1 / den rounded (FP64).
-__device__ __forceinline__ double tile_div(double n, double den, double r) {
-    const double q = n * r;
-    const double e = __builtin_fma(-q, den, n);
-    return __builtin_amdgcn_div_fixup(__builtin_fma(e, r, q), den, n);
-}
-
 // The lane's part of a psi solve: psi, the link factors of a(c, j) and
 // b(c, j) (FP32: scaled by dt/dx^2, dt/dy^2; zero where the link touches no
 // material), those of b above row 0, and the diagonals. FP32 keeps
@@ -390,7 +379,7 @@ __device__ __forceinline__ cplx<R> tile_psi_node(const PsiSweepArgs<R> &A, const
         const R q0pr = cb * pp.re + sb * pp.im, q0pi = cb * pp.im - sb * pp.re;
         const R nre = rhs.re + A.dt * (A.idx2 * (m0r + p0r) + A.idy2 * (q0mr + q0pr));
         const R nim = rhs.im + A.dt * (A.idx2 * (m0i + p0i) + A.idy2 * (q0mi + q0pi));
-        return {tile_div(nre, den, t.rden[r]), tile_div(nim, den, t.rden[r])};
+        return {div_by(nre, den, t.rden[r]), div_by(nim, den, t.rden[r])};
     }
 }
 
@@ -618,8 +607,8 @@ __device__ __forceinline__ void tile_a_sweep(const ASweepArgs<R> &A, ATile<R, SH
             Tb *= (j < 0 || j >= Ny - 1) ? R(0) : R(1);
         }
         if constexpr (std::is_same<R, double>::value) {
-            va = tile_div(t.Sa[r] + Ka * Ta, A.den_a, rden_a);
-            vb = tile_div(t.Sb[r] + Kb * Tb, A.den_b, rden_b);
+            va = div_by(t.Sa[r] + Ka * Ta, A.den_a, rden_a);
+            vb = div_by(t.Sb[r] + Kb * Tb, A.den_b, rden_b);
         } else {
             // in_vgpr: the change below is that of the rounded values (an fma
             // of the unrounded product would be off by up to half an ulp,
