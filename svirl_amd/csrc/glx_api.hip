@@ -153,6 +153,7 @@ int glx_init(int device) {
     e.stream = g_ctx.stream;
     e.partials = (double *)p; p += partials;
     e.result = (double *)p; p += result;
+    e.ticket = (unsigned *)(e.result + 63);  // the results take 32 at most
     e.arrive = (unsigned long long *)p; p += arrive;
     e.rel = (unsigned long long *)p; p += rel;
     e.chk = (unsigned long long *)p; p += chk;
@@ -164,6 +165,8 @@ int glx_init(int device) {
     if ((st = hipHostMalloc((void **)&e.energy_host, 64, hipHostMallocDefault)) != hipSuccess)
         return check_hip(st, "hipHostMalloc(energy)");
     e.energy_host[0] = 0.0;
+    if ((st = hipHostGetDevicePointer((void **)&e.energy_dev, e.energy_host, 0)) != hipSuccess)
+        return check_hip(st, "hipHostGetDevicePointer(energy)");
     if ((st = hipEventCreateWithFlags(&e.ev_energy, hipEventDisableTiming)) != hipSuccess)
         return check_hip(st, "hipEventCreate");
     if (!g_scratch_dev[device]) {  // with `device` current (hipSetDevice above)

@@ -25,7 +25,8 @@ namespace glx {
 // workgroups, the partials' capacity). On small grids a pass lasts as long as
 // a wave's rows, one after the other; the rows above and below that every
 // wave reads besides its own cost nothing while the chip is not full. Per
-// iteration of the FP32-mixed CG, kappa < inf, with 16 rows / one / this rule:
+// iteration of the FP32-mixed CG, kappa < inf, with 16 rows / one / this rule (and a kernel of
+// its own for the sums of a gradient pass):
 // 129^2 87 / 48 / 48 us, 385^2 89 / 54 / 54, 1025^2 108 / 100 / 86 (more waves
 // leave more partial sums to reduce), 2049^2 228 with any. FP64 keeps 16 rows,
 // and with them the order of its sums: its line search, on the host by the
@@ -63,7 +64,8 @@ template <typename R, bool withA, bool UPD>
 __global__ void __launch_bounds__(256) k_cg_grad_rows(Geo g, R kappa2, R eps, const R *eps_map, R H, const uint8_t *mt,
                                                       const cplx<R> *psi, const R *abei, const R *ab, cplx<R> *jac,
                                                       const cplx<R> *jac_prev, R *jacA, const R *jacA_prev,
-                                                      double *partials, StateUpdate<R> S, const double *alpha, long W) {
+                                                      double *partials, StateUpdate<R> S, const double *alpha, long W,
+                                                      GradFinish F) {
     constexpr int B = CGRows<R>::B;
     const GeoR<R> q(g);
     if constexpr (UPD) {
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(256) k_cg_grad_rows(Geo g, R kappa2, R eps, co
         const long w = (long)xcd_block() * (blockDim.x / WAVE) + wave_id();
         if (w < W) for_rows_rm<1>(g.Nx, g.Ny, w, W, [&](int s, int ja, int jb) { body(s, ja, jb, true); });
     }
-    block_store_partials<5>(acc, partials);
+    finish_gradient<R>(acc, partials, F);
 }
 
 // The line-search coefficients of the new direction d = beta d_old - g,

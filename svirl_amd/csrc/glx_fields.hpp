@@ -922,18 +922,65 @@ __global__ void __launch_bounds__(256) k_cg_gradient_pass(Geo g, R kappa2, R eps
     block_store_partials<5>(acc, partials);
 }
 
-// Finish of k_cg_gradient_pass: out[0] = dxdy * F (to be read by the host);
-// beta_next[0..1] = max(num/den, 0) for psi and A, in FP64 rounded to the
-// working precision (cg.py:422-449), left in device memory for the next
-// direction update.
+// Where a gradient pass leaves its sums: the free energy (the first sum
+// times dxdy) in out[0], and beta_next[0..1] = max(num/den, 0) for psi and A,
+// in FP64 rounded to the working precision (cg.py:422-449), in device memory
+// for the next direction update. `ticket` counts the launch's workgroups and
+// is zero between launches.
+struct GradFinish {
+    double dxdy;
+    double *out, *beta_next;
+    unsigned *ticket;
+};
+
+// The end of a gradient pass: every workgroup stores its five partial sums
+// past the caches and takes a ticket, and the last one reduces them all, in
+// the order of reduce_partials. (A kernel of its own for that takes 4.4 us
+// and the gap before it, and a copy of the energy to the host as much again;
+// on 129 x 129, psi only, 20 iterations of the FP32 CG took 768 us that way and
+// take 702.)
 template <typename R>
-__global__ void __launch_bounds__(256) k_cg_gradient_finish(const double *partials, int nb, double dxdy, double *out, double *beta_next) {
-    __shared__ double v[5];
-    reduce_partials<5>(partials, nb, v);
+__device__ __forceinline__ void finish_gradient(double (&acc)[5], double *partials, const GradFinish &F) {
+    __shared__ double lds[RED_BLOCK / WAVE * 5], v[5];
+    __shared__ int last;
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE, nw = blockDim.x / WAVE, nb = gridDim.x;
+    auto gather = [&](double (&a)[5]) {  // workgroup sums, thread k < 5 returns the k-th
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const double s = wave_sum(a[k]);
+            if (lane == 0) lds[wid * 5 + k] = s;
+        }
+        __syncthreads();
+        double s = 0.0;
+        if (threadIdx.x < 5)
+            for (int w = 0; w < nw; ++w) s += lds[w * 5 + threadIdx.x];
+        return s;
+    };
+    const double mine = gather(acc);
+    if (threadIdx.x < 5)
+        __hip_atomic_store(partials + (long)blockIdx.x * 5 + threadIdx.x, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);  // the sums are in memory before the ticket is taken
+    __syncthreads();
     if (threadIdx.x == 0) {
-        out[0] = v[0] * dxdy;
-        beta_next[0] = double(R(fmax(v[1] / v[2], 0.0)));
-        beta_next[1] = double(R(fmax(v[3] / v[4], 0.0)));
+        const unsigned t = __hip_atomic_fetch_add(F.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = t + 1 == (unsigned)nb;
+    }
+    __syncthreads();
+    if (!last) return;
+    double all[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k)
+            all[k] += __hip_atomic_load(partials + (long)b * 5 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const double total = gather(all);
+    if (threadIdx.x < 5) v[threadIdx.x] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(F.out, v[0] * F.dxdy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        F.beta_next[0] = double(R(fmax(v[1] / v[2], 0.0)));
+        F.beta_next[1] = double(R(fmax(v[3] / v[4], 0.0)));
+        __hip_atomic_store(F.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 

@@ -36,9 +36,11 @@ struct Env {
     // memory passes of the last td_run (psi passes, psi redone, A passes, A
     // redone, A passes with one more A buffer), or NULL
     int *passes;
-    // asynchronous energy readback of glx_cg_update_gradient_pass: the copy
-    // goes to pinned host memory and ev_energy is recorded after it
-    double *energy_host;
+    // asynchronous energy readback of glx_cg_update_gradient_pass: the pass
+    // writes it to pinned host memory (energy_dev is its device address) and
+    // ev_energy is recorded after it
+    double *energy_host, *energy_dev;
+    unsigned *ticket;        // workgroup count of a gradient pass, zero between launches
     hipEvent_t ev_energy;
     // the next TD run (single or batched) starts with the barrier error flag
     // raised, so every team leaves at its first barrier as after a timeout

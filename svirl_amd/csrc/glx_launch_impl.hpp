@@ -1550,7 +1550,7 @@ template <typename R>
 static int gradient_pass_launch(const Env &e, glx_grid g, double kappa2, double eps, const void *eps_map, double H,
                                 const uint8_t *mt, const void *psi, const void *abei, const void *ab, void *jac,
                                 const void *jac_prev, void *jacA, const void *jacA_prev, const StateUpdate<R> &S,
-                                const double *alpha, int *nb_out) {
+                                const double *alpha, double *out, double *beta_next) {
     const bool withA = kappa2 > 0.0;  // the psi Jacobian reads A in both cases
     const bool upd = S.dpsi != nullptr;
     const Geo G = make_geo(g.Nx, g.Ny, g.dx, g.dy);
@@ -1563,7 +1563,7 @@ static int gradient_pass_launch(const Env &e, glx_grid g, double kappa2, double 
     // overlap their loads, not in bytes)
     const long W = fit_row_waves(fn, cg_row_waves<R>(g.Nx, g.Ny), e.num_cus, 2);
     const int nb = (int)((W + 3) / 4);
-    *nb_out = nb;
+    const GradFinish F{double(R(g.dx)) * double(R(g.dy)), out, beta_next, e.ticket};
     const R k2 = R(kappa2), ep = R(eps), h = R(H);
     const R *em = (const R *)eps_map, *ae = (const R *)abei, *a = (const R *)ab;
     const cplx<R> *p = (const cplx<R> *)psi, *jp = (const cplx<R> *)jac_prev;
@@ -1572,16 +1572,16 @@ static int gradient_pass_launch(const Env &e, glx_grid g, double kappa2, double 
     const R *jAp = withA ? (const R *)jacA_prev : nullptr;
     if (withA && upd)
         hipLaunchKernelGGL((k_cg_grad_rows<R, true, true>), dim3(nb), dim3(RED_BLOCK), 0, e.stream, G, k2, ep, em, h, mt,
-                           p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W);
+                           p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W, F);
     else if (withA)
         hipLaunchKernelGGL((k_cg_grad_rows<R, true, false>), dim3(nb), dim3(RED_BLOCK), 0, e.stream, G, k2, ep, em, h,
-                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W);
+                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W, F);
     else if (upd)
         hipLaunchKernelGGL((k_cg_grad_rows<R, false, true>), dim3(nb), dim3(RED_BLOCK), 0, e.stream, G, k2, ep, em, h,
-                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W);
+                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W, F);
     else
         hipLaunchKernelGGL((k_cg_grad_rows<R, false, false>), dim3(nb), dim3(RED_BLOCK), 0, e.stream, G, k2, ep, em, h,
-                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W);
+                           mt, p, ae, a, jc, jp, jA, jAp, e.partials, S, alpha, W, F);
     GLX_LAUNCH_CHECK("k_cg_grad_rows");
     return GLX_OK;
 }
@@ -1602,20 +1602,13 @@ int L<R>::cg_update_gradient_pass(const Env &e, glx_grid g, double kappa2, doubl
     if (psi_out == psi || psi_out == dpsi || (dab && (ab_out == ab || ab_out == dab)))
         return set_error(GLX_E_ARG, "glx_cg_update_gradient_pass: the updated state needs buffers of its own");
     const StateUpdate<R> S{(const cplx<R> *)dpsi, (const R *)dab, (cplx<R> *)psi_out, (R *)ab_out, R(0), R(0)};
-    int nb = 0;
+    // asynchronous (F NULL): the pass writes the energy to pinned memory;
+    // glx_cg_energy_wait waits for the pass only, not for work enqueued after it
     int rc = gradient_pass_launch<R>(e, g, kappa2, eps, eps_map, H, mt, psi, abei, ab, jac, jac_prev, jacA, jacA_prev,
-                                     S, alpha_dev, &nb);
+                                     S, alpha_dev, F ? e.result : e.energy_dev, beta_next_dev);
     if (rc) return rc;
-    const double dxdy = double(R(g.dx)) * double(R(g.dy));
-    hipLaunchKernelGGL(k_cg_gradient_finish<R>, dim3(1), dim3(RED_BLOCK), 0, e.stream, e.partials, nb, dxdy, e.result,
-                       beta_next_dev);
-    GLX_LAUNCH_CHECK("k_cg_gradient_finish");
     if (F) return fetch_result(e, F, 1);
-    // asynchronous: the energy lands in pinned memory; glx_cg_energy_wait
-    // waits for this copy only, not for work enqueued after it
-    hipError_t st = hipMemcpyAsync(e.energy_host, e.result, sizeof(double), hipMemcpyDeviceToHost, e.stream);
-    if (st == hipSuccess) st = hipEventRecord(e.ev_energy, e.stream);
-    return check_hip(st, "glx_cg_update_gradient_pass energy readback");
+    return check_hip(hipEventRecord(e.ev_energy, e.stream), "glx_cg_update_gradient_pass energy");
 }
 
 template <typename R>
@@ -1627,14 +1620,9 @@ int L<R>::cg_gradient_pass(const Env &e, glx_grid g, double kappa2, double eps, 
         return set_error(GLX_E_ARG, "glx_cg_gradient_pass: invalid arguments");
     if (withA && (!(abei || ab) || !jacA || !jacA_prev))
         return set_error(GLX_E_ARG, "glx_cg_gradient_pass: finite kappa needs the vector potential and its Jacobians");
-    int nb = 0;
     int rc = gradient_pass_launch<R>(e, g, kappa2, eps, eps_map, H, mt, psi, abei, ab, jac, jac_prev, jacA, jacA_prev,
-                                     StateUpdate<R>{}, nullptr, &nb);
+                                     StateUpdate<R>{}, nullptr, e.result, beta_next_dev);
     if (rc) return rc;
-    const double dxdy = double(R(g.dx)) * double(R(g.dy));
-    hipLaunchKernelGGL(k_cg_gradient_finish<R>, dim3(1), dim3(RED_BLOCK), 0, e.stream, e.partials, nb, dxdy, e.result,
-                       beta_next_dev);
-    GLX_LAUNCH_CHECK("k_cg_gradient_finish");
     return fetch_result(e, F, 1);
 }
 
