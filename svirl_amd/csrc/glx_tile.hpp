@@ -327,11 +327,14 @@ __device__ __forceinline__ void tile_psi_load(const PsiSweepArgs<R> *Ap, const c
         const bool cellc = tile_cell(has_mt, mc[r], hasa, j, Ny), leftc = shfl_up1((int)cellc) != 0;
         const bool in = col && j >= 0 && j < Ny;
         t.p[r] = {in ? t.p[r].re : R(0), in ? t.p[r].im : R(0)};
-        const R den = psi_den(A, t.p[r], has_em ? ev[r] : A.eps, leftm, leftc, cellm, cellc);
-        // outside the material the sweep gives 0: all four link factors are
-        // zero there, and so is the right-hand side
+        // outside the material (and beyond the grid) the sweep gives 0: all
+        // four link factors are zero there, so is the right-hand side, and
+        // the diagonal is 1 (with eps it would be 0 where dt eps = 1, and
+        // 0 / 0 would spread from there)
         const bool inside = leftm || leftc || cellm || cellc;
         const cplx<R> rh = {inside ? t.p[r].re : R(0), inside ? t.p[r].im : R(0)};
+        const R e = has_em ? ev[r] : A.eps;
+        const R den = psi_den(A, rh, inside ? e : R(0), leftm, leftc, cellm, cellc);
         if constexpr (FOLD) {
             t.rden[r] = den;
             t.rd[r] = {fmaf(rh.re, den, -t.p[r].re), fmaf(rh.im, den, -t.p[r].im)};
