@@ -16,18 +16,30 @@
 // The FP64 arithmetic is that of the row-marching passes (psi_rows, a_rows):
 // results and every sweep count equal theirs to the bit.
 //
-// FP32 psi solves carry the change d of a sweep and the sum D of the changes
-// instead of psi and its right-hand side: the solve is linear in psi, so
-// d' = M d, and psi^{n+1} = psi^n + D. That costs the same registers and
-// instructions, D is rounded at the size of a step's change (a hundredth of
-// psi's), and the stop rule's 1e-6 is tested on values whose own rounding is
-// 1e-13, where the difference of two rounded iterates is off by up to 1e-7
-// and makes about 2 of 100 solves go a sweep too far.
+// FP32 psi solves carry, from their sweep PSI_TURN on, the change d of a sweep
+// and the sum D of the changes instead of psi and its right-hand side: the
+// solve is linear in psi, so d' = M d, and psi^{n+1} is the iterate at the
+// turn plus D. That costs the same registers and instructions, D is rounded at
+// the size of the changes that are left, and the stop rule's 1e-6 is tested on
+// values whose own rounding is 1e-13, where the difference of two rounded
+// iterates is off by up to 1e-7 and makes about 2 of 100 solves go a sweep too
+// far. The first sweeps carry psi itself because a step may shrink psi by
+// much (4 times a step where A outgrows the vortices): changes summed from
+// psi^n are rounded at its size, not psi^{n+1}'s, and after 20 such steps the
+// error against 64 bits was 1.6 times that of the row-marching solves, which
+// carry psi throughout (513^2: 5.8e-7 against 3.4e-7; with the turn 3.5e-7).
+// Over 70 runs of 10 steps on 65 x 65 to 1025 x 1025: tiles 2.4e-7 at most and
+// 2.0e-7 in the mean, no sweep count off; rows 8.2e-7, 2.5e-7 and 19 of 700 off.
 #pragma once
 
 #include "glx_td.hpp"
 
 namespace glx {
+
+// A FP32 psi solve carries changes from this sweep on; from its first one if
+// the previous step took PSI_FEW sweeps or fewer (psi hardly changes then,
+// and the stop rule is met among the first sweeps).
+constexpr int PSI_TURN = 2, PSI_FEW = 4;
 
 // A tile shape: NW waves of NR rows each, halo H.
 template <int NR_, int H_, int NW_> struct TileOf {
@@ -63,6 +75,11 @@ template <typename R, typename SH> struct TileLds {
     static constexpr int KR = std::is_same<R, double>::value ? NR : 1;
     cplx<R> rhs[KW][KR][WAVE];
     R den[KW][KR][WAVE];
+    // FP32: the right-hand side of every node up to the turn, psi at the turn
+    // from there on
+    static constexpr int TW = std::is_same<R, double>::value ? 1 : NW;
+    static constexpr int TR = std::is_same<R, double>::value ? 1 : NR;
+    cplx<R> base[TW][TR][WAVE];
     unsigned bits[NW], all;
     int fail;
 };
@@ -218,8 +235,8 @@ template <> struct TileSinCos<double> {
 // The lane's part of a psi solve: psi, the link factors of a(c, j) and
 // b(c, j) (FP32: scaled by dt/dx^2, dt/dy^2; zero where the link touches no
 // material), those of b above row 0, and the diagonals. FP32 keeps
-// 1/den, and the change of the last sweep in p (psi^n before the first) and
-// the sum of all in rd (rhs/den - psi^n before the first); FP64 1/den and, in
+// 1/den, and psi in p and rhs/den in rd up to the turn, from there on the
+// change of the last sweep in p and the sum of all in rd; FP64 1/den and, in
 // LDS, rhs and den.
 template <typename R, typename SH> struct PsiTile {
     static constexpr int NR = SH::NR;
@@ -337,7 +354,8 @@ __device__ __forceinline__ void tile_psi_load(const PsiSweepArgs<R> *Ap, const c
         const R den = psi_den(A, rh, inside ? e : R(0), leftm, leftc, cellm, cellc);
         if constexpr (FOLD) {
             t.rden[r] = den;
-            t.rd[r] = {fmaf(rh.re, den, -t.p[r].re), fmaf(rh.im, den, -t.p[r].im)};
+            t.rd[r] = {rh.re * den, rh.im * den};
+            S.base[X.w][r][X.lane] = rh;
         } else {
             t.rden[r] = R(1) / den;
             S.rhs[X.w][r][X.lane] = rh;
@@ -349,27 +367,27 @@ __device__ __forceinline__ void tile_psi_load(const PsiSweepArgs<R> *Ap, const c
     }
 }
 
+// U(-dy b) psi of a node: its part in the sum of the node above it.
+template <typename R> __device__ __forceinline__ cplx<R> tile_psi_up(const cplx<R> &p, R cb, R sb) {
+    return {cb * p.re - sb * p.im, cb * p.im + sb * p.re};
+}
+
 // One node: psi^{j+1} (FP32: its neighbours' part in it) from its own value,
-// the rows below and above it (pm, pp) and the lanes either side; (cm, sm)
-// are the factors of the link below.
+// the part m of the row below, the row above (pp) and the lanes either side.
 template <typename R, typename SH>
 __device__ __forceinline__ cplx<R> tile_psi_node(const PsiSweepArgs<R> &A, const PsiTile<R, SH> &t, int r,
-                                                 const cplx<R> &p, const cplx<R> &pm, const cplx<R> &pp, R cm, R sm,
+                                                 const cplx<R> &p, const cplx<R> &m, const cplx<R> &pp,
                                                  const cplx<R> &rhs, R den) {
     const R ca = t.ca[r], sa = t.sa[r], cb = t.cb[r], sb = t.sb[r];
     const R pr_re = shfl_dn1(p.re), pr_im = shfl_dn1(p.im);
     // this lane's part in the sum of the lane to the right
     const R l_re = ca * p.re - sa * p.im, l_im = ca * p.im + sa * p.re;
     if constexpr (std::is_same<R, float>::value) {
-        float re = ca * pr_re, im = ca * pr_im;
+        float re = fmaf(ca, pr_re, m.re), im = fmaf(ca, pr_im, m.im);
         re = fmaf(sa, pr_im, re);
         im = fmaf(-sa, pr_re, im);
         re += shfl_up1(l_re);
         im += shfl_up1(l_im);
-        re = fmaf(cm, pm.re, re);
-        im = fmaf(cm, pm.im, im);
-        re = fmaf(-sm, pm.im, re);
-        im = fmaf(sm, pm.re, im);
         re = fmaf(cb, pp.re, re);
         im = fmaf(cb, pp.im, im);
         re = fmaf(sb, pp.im, re);
@@ -378,10 +396,9 @@ __device__ __forceinline__ cplx<R> tile_psi_node(const PsiSweepArgs<R> &A, const
     } else {
         const R m0r = shfl_up1(l_re), m0i = shfl_up1(l_im);
         const R p0r = ca * pr_re + sa * pr_im, p0i = ca * pr_im - sa * pr_re;
-        const R q0mr = cm * pm.re - sm * pm.im, q0mi = cm * pm.im + sm * pm.re;
         const R q0pr = cb * pp.re + sb * pp.im, q0pi = cb * pp.im - sb * pp.re;
-        const R nre = rhs.re + A.dt * (A.idx2 * (m0r + p0r) + A.idy2 * (q0mr + q0pr));
-        const R nim = rhs.im + A.dt * (A.idx2 * (m0i + p0i) + A.idy2 * (q0mi + q0pi));
+        const R nre = rhs.re + A.dt * (A.idx2 * (m0r + p0r) + A.idy2 * (m.re + q0pr));
+        const R nim = rhs.im + A.dt * (A.idx2 * (m0i + p0i) + A.idy2 * (m.im + q0pi));
         return {div_by(nre, den, t.rden[r]), div_by(nim, den, t.rden[r])};
     }
 }
@@ -415,14 +432,14 @@ __device__ __forceinline__ void tile_edges_out(TileLds<R, SH> &S, int par, const
     S.edge[par][2 * X.w + 2][X.lane] = hi;
 }
 
-// n psi sweeps on the tile, the first of them the solve's first one or not
-// (FP32); bit s of the result: sweep s left a change of at
-// least thr at some node of the tile that belongs to this wave. `par` is the
+// n psi sweeps on the tile, the first of them the solve's sweep j (FP32 carries
+// changes from sweep `turn` on); bit s of the result: sweep s left a change of
+// at least thr at some node of the tile that belongs to this wave. `par` is the
 // LDS copy the first sweep reads (the caller's edges are there, behind a
 // barrier) and, on return, the one to be used next.
 template <typename R, typename SH>
 __device__ __forceinline__ unsigned tile_psi_sweeps(const PsiSweepArgs<R> *Ap, PsiTile<R, SH> &t, TileLds<R, SH> &S,
-                                                    const TileCtx &X, int n, R thr, int &par_, bool first) {
+                                                    const TileCtx &X, int n, R thr, int &par_, int j, int turn) {
     constexpr int NR = SH::NR;
     int par = uniform(par_);
     constexpr bool F64 = std::is_same<R, double>::value;
@@ -430,36 +447,42 @@ __device__ __forceinline__ unsigned tile_psi_sweeps(const PsiSweepArgs<R> *Ap, P
     unsigned bits = 0u;
     const cplx<R>(*rl)[WAVE] = S.rhs[F64 ? X.w : 0];
     const R(*dl)[WAVE] = S.den[F64 ? X.w : 0];
-    for (int s = 0; s < n; ++s) {
+    auto sweep = [&](auto changes, int s, bool first) {
+        constexpr bool CHANGES = decltype(changes)::value;
         // the rows above and below the wave's (unknown beyond the tile)
         const cplx<R> up = S.edge[par][2 * X.w][X.lane], dn = S.edge[par][2 * X.w + 3][X.lane];
         TileRes<R> res{R(0), R(0), R(0), R(0)};
-        auto node = [&](int r, const cplx<R> &p, const cplx<R> &pm, const cplx<R> &pp, R cm, R sm) {
-            const cplx<R> q = tile_psi_node<R, SH>(A, t, r, p, pm, pp, cm, sm, rl[F64 ? r : 0][X.lane],
+        auto node = [&](int r, const cplx<R> &p, const cplx<R> &m, const cplx<R> &pp) {
+            const cplx<R> q = tile_psi_node<R, SH>(A, t, r, p, m, pp, rl[F64 ? r : 0][X.lane],
                                                  dl[F64 ? r : 0][X.lane]);
-            if constexpr (F64) {
-                res.template add<SH>(r, fmax(fabs(q.re - p.re), fabs(q.im - p.im)));
-                return q;
-            } else {
-                t.rd[r] = {fmaf(q.re, t.rden[r], t.rd[r].re), fmaf(q.im, t.rden[r], t.rd[r].im)};
-                const cplx<R> d = {q.re * t.rden[r], q.im * t.rden[r]};
-                res.template add<SH>(r, fmax(fabs(d.re), fabs(d.im)));
-                return d;
+            cplx<R> v = q, d = {q.re - p.re, q.im - p.im};
+            if constexpr (!F64) {
+                v = {fmaf(q.re, t.rden[r], t.rd[r].re), fmaf(q.im, t.rden[r], t.rd[r].im)};
+                d = CHANGES ? cplx<R>{q.re * t.rden[r], q.im * t.rden[r]} : cplx<R>{v.re - p.re, v.im - p.im};
+                if constexpr (CHANGES) {
+                    t.rd[r] = v;
+                    v = d;
+                }
             }
+            res.template add<SH>(r, fmax(fabs(d.re), fabs(d.im)));
+            return v;
         };
         // rows 1 .. NR-1, then row 0: `up` and `dn` have the middle rows to
-        // arrive in
-        const cplx<R> old0 = t.p[0], old1 = t.p[1];
-        cplx<R> prev = old0;
+        // arrive in. A row's part in the sum of the next is formed before its
+        // new value, which then takes its place in the registers (formed with
+        // the next row it keeps the old value alive, and the loop moves two
+        // registers a row: 24 of 384 instructions a sweep of 14 rows)
+        const cplx<R> old1 = t.p[1];
+        cplx<R> m = tile_psi_up(t.p[0], t.cb[0], t.sb[0]);
 #pragma unroll
         for (int r = 1; r < NR; ++r) {
-            const cplx<R> cur = t.p[r];
-            t.p[r] = node(r, cur, prev, r + 1 < NR ? t.p[r + 1 < NR ? r + 1 : r] : dn, t.cb[r - 1], t.sb[r - 1]);
-            prev = cur;
+            const cplx<R> cur = t.p[r], below = m;
+            if (r + 1 < NR) m = tile_psi_up(cur, t.cb[r], t.sb[r]);
+            t.p[r] = node(r, cur, below, r + 1 < NR ? t.p[r + 1 < NR ? r + 1 : r] : dn);
         }
-        t.p[0] = node(0, old0, up, old1, t.cbu, t.sbu);
-        if constexpr (!F64) {
-            if (first && s == 0) {  // the first change has the own value's part too
+        t.p[0] = node(0, t.p[0], tile_psi_up(up, t.cbu, t.sbu), old1);
+        if constexpr (CHANGES) {
+            if (first) {  // the first change has the own value's part too
                 res = {R(0), R(0), R(0), R(0)};
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
@@ -473,7 +496,22 @@ __device__ __forceinline__ unsigned tile_psi_sweeps(const PsiSweepArgs<R> *Ap, P
         const bool open = X.own<SH>(A.Nx) && res.template of<SH>(X) >= thr;
         bits |= __ballot(open) != 0ull ? 1u << s : 0u;
         __syncthreads();
-    }
+    };
+    int s = 0;
+    for (; s < n && (F64 || j + s < turn); ++s) sweep(std::false_type{}, s, false);
+    if constexpr (!F64)
+        for (; s < n; ++s) {
+            const bool first = j + s == turn;
+            if (first) {  // rhs/den - psi, rounded once
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const cplx<R> rh = S.base[X.w][r][X.lane];
+                    S.base[X.w][r][X.lane] = t.p[r];
+                    t.rd[r] = {fmaf(rh.re, t.rden[r], -t.p[r].re), fmaf(rh.im, t.rden[r], -t.p[r].im)};
+                }
+            }
+            sweep(std::true_type{}, s, first);
+        }
     par_ = par;
     return bits;
 }
@@ -694,17 +732,15 @@ __device__ __forceinline__ void tile_psi_publish(int Nx, int Ny, cplx<R> *out, c
             st_shared_mem(out + (size_t)Nx * (X.j0 + r) + cc, p[r]);
 }
 
-// psi^{n+1} = psi^n + D of a FP32 solve at the nodes of the tile.
+// psi of a FP32 solve past its turn at the nodes of the tile.
 template <typename R, typename SH>
-__device__ __forceinline__ void tile_psi_total(int Nx, int Ny, const cplx<R> *psi, const TileCtx &X0,
-                                               const PsiTile<R, SH> &t, cplx<R> (&p)[SH::NR]) {
-    constexpr int NR = SH::NR;
-    const TileCtx X = X0.fresh();
-    const uint32_t oc = X.cc(Nx) * (uint32_t)sizeof(R);
+__device__ __forceinline__ void tile_psi_total(const TileLds<R, SH> &S, const TileCtx &X, const PsiTile<R, SH> &t,
+                                               cplx<R> (&p)[SH::NR]) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) p[r] = ld_at(tile_row(psi, X.j0 + r, Ny, Nx), 2 * oc);
-#pragma unroll
-    for (int r = 0; r < NR; ++r) p[r] = {p[r].re + t.rd[r].re, p[r].im + t.rd[r].im};
+    for (int r = 0; r < SH::NR; ++r) {
+        const cplx<R> b = S.base[X.w][r][X.lane];
+        p[r] = {b.re + t.rd[r].re, b.im + t.rd[r].im};
+    }
 }
 template <typename R, typename SH>
 __device__ __forceinline__ void tile_a_publish(int Nx, int Ny, R *out, const TileCtx &X0, const ATile<R, SH> &t,
@@ -904,8 +940,8 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
             TileSched sc(pred, H, max_sweeps);
             unsigned bits = 0u;
             int nsw = 0, stop = 0;  // stop: the sweep a redone solve ends at
+            const int turn = pred > 0 && pred <= PSI_FEW ? 0 : PSI_TURN;
             bool again;
-            cplx<R> tot[NR];  // psi^{n+1} (FP32)
             do {
                 again = false;
                 tile_psi_load<R, SH>(&T->psi, arg(&T->P[uniform(pc)]), X, t, S);
@@ -914,15 +950,17 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                     tile_edges_out<R, SH>(S, par, X, t.p[0], t.p[NR - 1]);
                     __syncthreads();
                     const int n = uniform(min(sc.next - sc.j, H));
-                    bits |= tile_psi_sweeps<R, SH>(&T->psi, t, S, X, n, thr_psi, par, uniform(sc.j) == 0) << (sc.j - sc.j0);
+                    bits |= tile_psi_sweeps<R, SH>(&T->psi, t, S, X, n, thr_psi, par, uniform(sc.j), uniform(turn)) << (sc.j - sc.j0);
                     sc.j += n;
                     const bool check = uniform(sc.j) == uniform(sc.next);
                     cur = cur == o1 ? o2 : o1;
                     // FP32: all of psi^{n+1} goes out at a check, the ring of
-                    // changes where the solve goes on
+                    // psi or changes where the solve goes on
                     if (F64 || check) {
-                        if constexpr (!F64) tile_psi_total<R, SH>(Nx, Ny, arg(&T->P[uniform(pc)]), X, t, tot);
-                        const cplx<R>(&v)[NR] = F64 ? t.p : tot;
+                        cplx<R> v[NR];
+#pragma unroll
+                        for (int r = 0; r < NR; ++r) v[r] = t.p[r];
+                        if (!F64 && uniform(sc.j) > uniform(turn)) tile_psi_total<R, SH>(S, X, t, v);
                         tile_psi_publish<R, SH>(Nx, Ny, arg(&T->P[uniform(cur)]), X, v, check);
                     }
                     if (check) {
@@ -950,10 +988,7 @@ __device__ __forceinline__ void tile_run(const TDSolveArgs<R> *T, const TileSync
                 }
             } while (again);
             if (!ok) break;
-            if constexpr (!F64) {
-#pragma unroll
-                for (int r = 0; r < NR; ++r) t.p[r] = tot[r];
-            }
+            if (!F64 && uniform(nsw) > uniform(turn)) tile_psi_total<R, SH>(S, X, t, t.p);
             pred = nsw;
             if (threadIdx.x == 0 && tm.tx == 0 && tm.ty == 0) sweeps[(long)step * stride] = nsw;
         }
