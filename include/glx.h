@@ -167,24 +167,31 @@ typedef struct glx_batch_instance {
 } glx_batch_instance;
 
 /* Advance n instances by nsteps TD steps, each with its own stop rule and
- * sweep counts (as glx_td_run would alone). Instances whose nodes fit in
- * the registers of the GPU (up to about a million nodes) run all steps in
- * one launch with as many others as fit beside them. For larger ones every
+ * sweep counts (as glx_td_run would alone). With wg_per_cu 0, instances whose
+ * nodes fit in the registers of the GPU (up to about 1.3 million nodes in
+ * FP32, 1.0 million in FP64) run all steps in one launch with as many others
+ * as fit beside them. For larger ones, and with wg_per_cu > 0 for all, every
  * step is ONE persistent launch in which each instance is swept by its own
  * team of co-resident workgroups with team-local barriers; what follows is
  * about these. Teams are sized in proportion to each instance's wave-rows
  * times weight[i] (its relative sweeps per step, e.g. from an earlier run;
  * NULL = 1). With use_graph != 0, the step launches are captured once into
- * a HIP graph and replayed. wg_per_cu (co-resident workgroups per CU, 0 = as many as fit),
- * min_rows (fewest rows per wave when sizing teams, 0 = 16) and psi_depth
- * (sweeps per psi pass, 2..4, i.e. strips of 64 - 2*psi_depth columns;
- * 0 = 3) are the tunable tile shape; the results do not depend on them.
+ * a HIP graph and replayed. wg_per_cu (co-resident workgroups per CU, for
+ * instance fewer where the GPU is shared; 0 = as many as fit), min_rows
+ * (fewest rows per wave when sizing teams, 0 = 16) and psi_depth (sweeps per
+ * psi pass, 2..4, i.e. strips of 64 - 2*psi_depth columns; 0 = 3) are the
+ * tunable shape; the results do not depend on them (FP32: but for the
+ * rounding between the two forms that wg_per_cu 0 and > 0 select).
  * sweeps (host, nsteps*n*2 int32, may be NULL) receives (S_psi, S_A) per
  * step and instance. Instances must not share buffers; n must not exceed
  * the number of co-resident workgroups. */
 int glx_batch_td_run(int prec, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
                      int32_t use_graph, int32_t wg_per_cu, int32_t min_rows, const double *weight,
                      int32_t psi_depth);
+
+/* Which instances glx_batch_td_run would hold in registers (tiled[i] 1) and
+ * which it would sweep by teams (0), by their grids and p.solveA alone. */
+int glx_batch_td_tiled(int prec, const glx_batch_instance *inst, int32_t n, int32_t wg_per_cu, int32_t *tiled);
 
 /* Bytes of the fixed device scratch array behind glx_batch_td_run_noalloc. */
 #define GLX_NOALLOC_SCRATCH_BYTES (8u << 20)

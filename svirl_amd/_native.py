@@ -88,6 +88,7 @@ _PROTOS = {
     "glx_td_force_barrier_abort": [],
     "glx_batch_td_run": [c_int, ctypes.POINTER(BatchInstance), c_i32, c_i32, P_i32, c_i32, c_i32, c_i32, c_void_p,
                          c_i32],
+    "glx_batch_td_tiled": [c_int, ctypes.POINTER(BatchInstance), c_i32, c_i32, P_i32],
     "glx_batch_td_run_noalloc": [c_int, ctypes.POINTER(BatchInstance), c_i32, c_i32, P_i32, c_i32, c_i32, c_void_p,
                                  c_i32],
     "glx_batch_cg_run": [c_int, ctypes.POINTER(BatchCGInstance), c_i32, c_i32, c_double, c_i32, c_i32, c_i32],

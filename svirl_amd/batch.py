@@ -5,18 +5,21 @@ The reference runs one GLSolver per process, one time step at a time
 (each with its own grid, kappa, field, epsilon map and mask) advances
 together (glx_batch_td_run): every instance is swept by its own workgroups,
 so each keeps its own Jacobi sweep counts and stop rule, exactly as if it had
-been run alone. Instances of up to about a million nodes are held in
-registers and run all steps in one launch, as many at a time as fit.
+been run alone. Instances of up to about 1.3 million nodes in FP32 and 1.0
+million in FP64 are held in registers and run all steps in one launch, as many
+at a time as fit.
 
 Larger ones advance by one persistent launch per time step, replayed from a
-captured HIP graph, in teams of workgroups whose shape matters. That shape — sweeps per psi pass (the tile depth, which sets the
-strip width: 64 - 2 x depth columns per wave), fewest rows per wave when
-sizing the teams (the tile height) and workgroups per CU — is picked by an
-autotuner: the first steps of a run time candidate shapes on the real state
-(the results do not depend on the shape), one axis at a time from a default
-(coordinate descent: depth, then height, then occupancy, each axis keeping
-its fastest value), and the rest of the run uses the fastest; the choice is
-cached per batch signature. Teams are sized by each instance's wave-rows
+captured HIP graph, in teams of workgroups whose shape matters. That shape —
+sweeps per psi pass (the depth, which sets the strip width: 64 - 2 x depth
+columns per wave), fewest rows per wave when sizing the teams (the height) and
+workgroups per CU (0: as many as fit; a number puts every instance on teams) —
+is picked by an autotuner: the first steps
+of a run time candidate shapes on the real state (the results do not depend
+on the shape, FP32 but for rounding between registers and teams), one axis at
+a time from a default (coordinate descent: depth, then height, then occupancy,
+each axis keeping its fastest value), and the rest of the run uses the
+fastest; the choice is cached per batch signature. Teams are sized by each instance's wave-rows
 times its sweeps per step in the previous run, so instances that iterate
 more get more workgroups.
 
@@ -50,8 +53,9 @@ TUNE_RUNS = 1 + sum(len(v) - 1 for _, v in AXES)
 class BatchTD:
     """Advance a list of GLSolver objects together (FP32 or FP64, all the
     same). use_graph: replay the step launches from a HIP graph.
-    autotune: pick the tile shape on the first steps (AXES; needs
-    tune_need() steps of the first td() call).
+    autotune: pick the teams' shape on the first steps (AXES; needs
+    tune_need() steps of the first td() call). A shape of the caller's own,
+    (wg_per_cu, min_rows, psi_depth), can be put in `shape`.
     noalloc: run through glx_batch_td_run_noalloc (no device allocation per
     call, its workspace is the library's fixed scratch array; no graph)."""
 
@@ -75,6 +79,18 @@ class BatchTD:
     def tune_need(self):
         """Steps the autotuner takes from the first td() call."""
         return self.tune_steps * (TUNE_RUNS + 1) + 1
+
+    def on_teams(self, wg_per_cu=0):
+        """Which instances run on teams of workgroups rather than held in
+        registers."""
+        n = len(self.solvers)
+        arr = (BatchInstance * n)()
+        for I, s in zip(arr, self.solvers):
+            I.g = nat.Grid(int(s.cfg.Nx), int(s.cfg.Ny), float(s.cfg.dx), float(s.cfg.dy))
+            I.p.solveA = 1 if s.params.solveA else 0
+        tiled = (ctypes.c_int32 * n)()
+        nat.call("glx_batch_td_tiled", self.prec, arr, n, int(wg_per_cu), tiled)
+        return [not t for t in tiled]
 
     def _signature(self):
         return tuple((int(s.cfg.Nx), int(s.cfg.Ny), bool(s.params.solveA)) for s in self.solvers) + (self.prec,)

@@ -339,6 +339,10 @@ int glx_batch_td_run(int prec, glx_batch_instance *inst, int32_t n, int32_t nste
                                     psi_depth, ws));
 }
 
+int glx_batch_td_tiled(int prec, const glx_batch_instance *inst, int32_t n, int32_t wg_per_cu, int32_t *tiled) {
+    GLX_DISPATCH(prec, batch_td_tiled(g_ctx.env, inst, n, wg_per_cu, tiled));
+}
+
 int glx_batch_td_run_noalloc(int prec, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
                              int32_t wg_per_cu, int32_t min_rows, const double *weight, int32_t psi_depth) {
     GLX_REQUIRE_INIT();

@@ -868,6 +868,34 @@ static int plan_tile_bins(const Env &e, const glx_batch_instance *inst, const st
     return GLX_OK;
 }
 
+// The launches of a batch's instances, those without (0) and with (1) A apart,
+// and the instances no tile shape holds.
+template <typename R>
+static int plan_batch_tiles(const Env &e, const glx_batch_instance *inst, int32_t n, std::vector<TileBin> (&bins)[2],
+                            std::vector<int> &left) {
+    std::vector<int> todo[2];
+    for (int i = 0; i < n; ++i) todo[inst[i].p.solveA ? 1 : 0].push_back(i);
+    double cost = 0.0;
+    int rc = plan_tile_bins<R, false>(e, inst, todo[0], &cost, bins[0], left);
+    if (!rc) rc = plan_tile_bins<R, true>(e, inst, todo[1], &cost, bins[1], left);
+    return rc;
+}
+
+template <typename R>
+int L<R>::batch_td_tiled(const Env &e, const glx_batch_instance *inst, int32_t n, int32_t wg_per_cu, int32_t *tiled) {
+    if (!inst || n < 1 || !tiled) return set_error(GLX_E_ARG, "glx_batch_td_tiled: invalid arguments");
+    for (int i = 0; i < n; ++i)
+        if (!grid_ok(inst[i].g)) return set_error(GLX_E_ARG, "glx_batch_td_tiled: instance %d: invalid grid", i);
+    std::fill(tiled, tiled + n, wg_per_cu > 0 ? 0 : 1);
+    if (wg_per_cu > 0) return GLX_OK;
+    std::vector<TileBin> bins[2];
+    std::vector<int> left;
+    const int rc = plan_batch_tiles<R>(e, inst, n, bins, left);
+    if (rc) return rc;
+    for (int i : left) tiled[i] = 0;
+    return GLX_OK;
+}
+
 // Zero the words of one launch's tiles; the error flag is set with the
 // batch's first launch (err0 >= 0) only.
 static __global__ void k_batch_tile_reset(TileSync ts, int nwg, int ngrp, int err0) {
@@ -886,12 +914,8 @@ template <typename R>
 static int batch_run_tiles(const Env &e, glx_batch_instance *inst, int32_t n, int32_t nsteps, int32_t *sweeps,
                            const Workspace &ws, std::vector<int> *left) {
     constexpr bool G = RunForm<R>::has_gauge;
-    std::vector<TileBin> bins[2];  // without, with A
-    std::vector<int> todo[2];
-    for (int i = 0; i < n; ++i) todo[inst[i].p.solveA ? 1 : 0].push_back(i);
-    double cost = 0.0;
-    int rc = plan_tile_bins<R, false>(e, inst, todo[0], &cost, bins[0], *left);
-    if (!rc) rc = plan_tile_bins<R, true>(e, inst, todo[1], &cost, bins[1], *left);
+    std::vector<TileBin> bins[2];
+    int rc = plan_batch_tiles<R>(e, inst, n, bins, *left);
     if (rc || (bins[0].empty() && bins[1].empty())) return rc;
     std::vector<TDSolveArgs<R>> args(n);
     std::vector<int> state(8 * (size_t)n, 0);
@@ -1054,6 +1078,8 @@ int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_
             if (any_A) return by_depth(std::true_type{});
         return by_depth(std::false_type{});
     };
+    // an explicit number of workgroups: teams, as in glx_td_run
+    if (wg_per_cu > 0) return rows(inst, n, sweeps, weight, false);
     // what the teams would refuse (too many instances, too little scratch) is refused
     int rc = rows(inst, n, nullptr, weight, true);
     if (rc) return rc;
