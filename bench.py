@@ -327,8 +327,8 @@ def run_batch(args):
     log(f"[c4] building {args.batch_n} Config 4 instances")
     sims = workloads.config4(n=args.batch_n, dtype=np.float32)
     nodes = sum(int(s.cfg.N) for s in sims)
-    b = BatchTD(sims, use_graph=True, autotune=True)
-    b.td(dt=0.1, Nt=b.tune_need())  # autotune on the first steps
+    b = BatchTD(sims, use_graph=True)
+    b.td(dt=0.1, Nt=b.tune_need())  # warmup, and the autotuner's steps where instances run on teams
     nat.call("glx_synchronize")
     t0 = time.perf_counter()
     b.td(dt=0.1, Nt=args.batch_steps)
@@ -336,7 +336,7 @@ def run_batch(args):
     tb = time.perf_counter() - t0
     rate_b = nodes * args.batch_steps / tb
     log(f"[c4] {len(sims)} instances, {nodes} nodes: {rate_b:.4g} node-steps/s batched "
-        f"({1e3 * tb / args.batch_steps:.3f} ms/step, shape {b.shape})")
+        f"({1e3 * tb / args.batch_steps:.3f} ms/step, {sum(b.on_teams())} on teams)")
     for s in sims:
         s.solve.td(dt=0.1, Nt=1)  # warm each instance's own launches
     nat.call("glx_synchronize")
@@ -350,8 +350,9 @@ def run_batch(args):
     sw = np.array([np.mean(np.array(s.solve._td.sweeps), axis=0) for s in sims])
     res = {"instances": len(sims), "nodes": nodes, "node_steps_per_s": rate_b, "ms_per_step": 1e3 * tb / args.batch_steps,
            "per_instance_node_steps_per_s": rate_s, "speedup_vs_per_instance": rate_b / rate_s,
+           "instances_on_teams": sum(b.on_teams()),
            "tuned_shape": {"wg_per_cu": b.shape[0], "min_rows": b.shape[1], "psi_depth": b.shape[2],
-                           "strip_columns": 64 - 2 * b.shape[2]},
+                           "strip_columns": 64 - 2 * b.shape[2]} if b.timings else None,
            "tuning_ms_per_step": {f"wg{k[0]},rows{k[1]},depth{k[2]}": v for k, v in b.timings.items()},
            "mean_sweeps_per_step": {"psi": float(sw[:, 0].mean()), "A": float(sw[:, 1].mean())},
            "dtype": "f32", "graph": True}

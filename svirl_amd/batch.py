@@ -14,7 +14,7 @@ captured HIP graph, in teams of workgroups whose shape matters. That shape —
 sweeps per psi pass (the depth, which sets the strip width: 64 - 2 x depth
 columns per wave), fewest rows per wave when sizing the teams (the height) and
 workgroups per CU (0: as many as fit; a number puts every instance on teams) —
-is picked by an autotuner: the first steps
+is picked by an autotuner where the batch has such instances: the first steps
 of a run time candidate shapes on the real state (the results do not depend
 on the shape, FP32 but for rounding between registers and teams), one axis at
 a time from a default (coordinate descent: depth, then height, then occupancy,
@@ -54,12 +54,13 @@ class BatchTD:
     """Advance a list of GLSolver objects together (FP32 or FP64, all the
     same). use_graph: replay the step launches from a HIP graph.
     autotune: pick the teams' shape on the first steps (AXES; needs
-    tune_need() steps of the first td() call). A shape of the caller's own,
-    (wg_per_cu, min_rows, psi_depth), can be put in `shape`.
+    tune_need() steps of the first td() call): None where the batch has
+    instances that run on teams, True always, False never. A shape of the
+    caller's own, (wg_per_cu, min_rows, psi_depth), can be put in `shape`.
     noalloc: run through glx_batch_td_run_noalloc (no device allocation per
     call, its workspace is the library's fixed scratch array; no graph)."""
 
-    def __init__(self, solvers, use_graph=True, autotune=True, tune_steps=4, noalloc=False):
+    def __init__(self, solvers, use_graph=True, autotune=None, tune_steps=4, noalloc=False):
         if not solvers:
             raise ValueError("BatchTD needs at least one solver")
         dt0 = solvers[0].cfg.dtype
@@ -69,7 +70,7 @@ class BatchTD:
         self.prec = nat.prec_of(dt0)
         self.noalloc = bool(noalloc)
         self.use_graph = bool(use_graph) and not self.noalloc
-        self.autotune = bool(autotune)
+        self.autotune = autotune if autotune is None else bool(autotune)
         self.tune_steps = int(tune_steps)
         self.shape = None
         self.timings = {}
@@ -157,7 +158,8 @@ class BatchTD:
         sig = self._signature()
         if self.shape is None:
             self.shape = _TUNED.get(sig)
-        if self.shape is None and self.autotune and Nt >= self.tune_need():
+        if (self.shape is None and self.autotune is not False and Nt >= self.tune_need()
+                and (self.autotune or any(self.on_teams()))):
             if self.weights is None:  # learn the per-instance sweep counts first
                 self._run(tds, self.tune_steps, DEFAULT_SHAPE)
                 done += self.tune_steps

@@ -1,6 +1,7 @@
 """Batched TD on teams of workgroups (wg_per_cu > 0, and instances that no
-register tile holds): graph replay, every pass depth, both precisions, and
-a timed-out run."""
+register tile holds): graph replay, every pass depth, both precisions, a
+timed-out run, and the autotuner, which times shapes only where instances run
+on teams."""
 import numpy as np
 import pytest
 
@@ -89,3 +90,28 @@ def test_teams_barrier_timeout_keeps_states():
     for gl, st in zip(sims, refs):
         assert [tuple(x) for x in gl.solve._td.sweeps] == st.sweeps
         assert np.max(np.abs(gl.flatten_array(gl.vars.order_parameter) - st.psi)) <= 1e-11
+
+
+def test_autotuner_leaves_batches_in_registers_alone():
+    from svirl_amd.batch import BatchTD
+    sims = [make(k, *c) for k, c in enumerate(CASES[:3])]
+    b = BatchTD(sims, tune_steps=1)
+    n = b.tune_need() + 1
+    b.td(dt=0.1, Nt=n)
+    assert b.timings == {}
+    assert all(len(gl.solve._td.sweeps) == n for gl in sims)
+
+
+def test_autotuner_times_shapes_of_teams():
+    """One instance on teams beside one in registers; the fields are those of
+    each alone."""
+    from svirl_amd.batch import BatchTD
+    sims, alone = ([make(1, *CASES[1]), big(np.float64, np.inf)] for _ in range(2))
+    b = BatchTD(sims, tune_steps=1)
+    n = b.tune_need() + 1
+    b.td(dt=0.1, Nt=n)
+    assert {k[2] for k in b.timings} == {2, 3, 4} and b.shape in b.timings
+    for gl, g1 in zip(sims, alone):
+        g1.solve.td(dt=0.1, Nt=n)
+        assert gl.solve._td.sweeps == g1.solve._td.sweeps
+        assert all(np.array_equal(x, y) for x, y in zip(fields(gl), fields(g1)))
