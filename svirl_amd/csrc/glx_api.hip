@@ -169,6 +169,12 @@ int glx_init(int device) {
         return check_hip(st, "hipHostGetDevicePointer(energy)");
     if ((st = hipEventCreateWithFlags(&e.ev_energy, hipEventDisableTiming)) != hipSuccess)
         return check_hip(st, "hipEventCreate");
+    if ((st = hipStreamCreateWithFlags(&e.side, hipStreamNonBlocking)) != hipSuccess)
+        return check_hip(st, "hipStreamCreate");
+    if ((st = hipEventCreateWithFlags(&e.ev_fork, hipEventDisableTiming)) != hipSuccess)
+        return check_hip(st, "hipEventCreate");
+    if ((st = hipEventCreateWithFlags(&e.ev_join, hipEventDisableTiming)) != hipSuccess)
+        return check_hip(st, "hipEventCreate");
     if (!g_scratch_dev[device]) {  // with `device` current (hipSetDevice above)
         void *sp = nullptr;
         if ((st = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch))) != hipSuccess)

@@ -42,6 +42,10 @@ struct Env {
     double *energy_host, *energy_dev;
     unsigned *ticket;        // workgroup count of a gradient pass, zero between launches
     hipEvent_t ev_energy;
+    // a second stream for a launch that runs beside one on `stream`, and the
+    // events it starts after and ends with
+    hipStream_t side;
+    hipEvent_t ev_fork, ev_join;
     // the next TD run (single or batched) starts with the barrier error flag
     // raised, so every team leaves at its first barrier as after a timeout
     // (glx_td_force_barrier_abort; cleared by that run)

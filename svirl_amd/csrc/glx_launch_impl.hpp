@@ -1111,15 +1111,15 @@ int L<R>::batch_td_run(const Env &e, glx_batch_instance *inst, int32_t n, int32_
 
 // ---- batched CG -----------------------------------------------------------------
 
-// `iters` iterations of n instances with NW waves each.
+// `iters` iterations of n instances with NW waves each, on `stream`.
 template <typename R, int LL, int NW>
-static int batch_cg_launch(const Env &e, const CGInst<R> *d_inst, double *d_state, int n, int iters, int max_iters,
+static int batch_cg_launch(const Env &e, hipStream_t stream, const CGInst<R> *d_inst, double *d_state, int n, int iters, int max_iters,
                            double rtol, int stall_iters) {
     int per_cu = 0;
     const hipError_t st = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_cg<R, LL, NW>, NW * WAVE, 0);
     if (st != hipSuccess) return check_hip(st, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     const int grid = std::max(1, std::min(n, per_cu * e.num_cus));
-    hipLaunchKernelGGL((k_batch_cg<R, LL, NW>), dim3(grid), dim3(NW * WAVE), 0, e.stream, d_inst, d_state, n, iters,
+    hipLaunchKernelGGL((k_batch_cg<R, LL, NW>), dim3(grid), dim3(NW * WAVE), 0, stream, d_inst, d_state, n, iters,
                        max_iters, rtol, stall_iters);
     GLX_LAUNCH_CHECK("k_batch_cg");
     return GLX_OK;
@@ -1145,10 +1145,13 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     CGInst<R> *d_inst = (CGInst<R> *)blk;
     double *d_state = (double *)(blk + s_inst);
     char *work = blk + s_inst + s_state;
-    // the ns small instances first, each at place at[i]
+    // the ns small instances first, each at place at[i] (all are where they
+    // take as many waves as the others)
     std::vector<int> at(n);
     int ns = 0, place = 0;
-    auto small = [&](int i) { return (long)inst[i].g.Nx * inst[i].g.Ny <= BATCH_CG_SMALL; };
+    auto small = [&](int i) {
+        return BatchCGWaves<R>::MOST == 4 || (long)inst[i].g.Nx * inst[i].g.Ny <= BATCH_CG_SMALL;
+    };
     for (int i = 0; i < n; ++i)
         if (small(i)) at[i] = ns++;
     place = ns;
@@ -1192,11 +1195,29 @@ static int batch_cg_form(const Env &e, glx_batch_cg_instance *inst, int32_t n, i
     for (int done = it_min; done < max_iters; done += chunk) {
         const int iters = std::min(chunk, max_iters - done);
         int rc = GLX_OK;
-        if (ns > 0) rc = batch_cg_launch<R, LL, 4>(e, d_inst, d_state, ns, iters, max_iters, rtol, stall_iters);
-        if (!rc && ns < n)
-            rc = batch_cg_launch<R, LL, BatchCGWaves<R>::MOST>(e, d_inst + ns, d_state + CG_NSTATE * ns, n - ns, iters,
-                                                              max_iters, rtol, stall_iters);
+        // a batch of both kinds: the small ones beside the others (ten of 60 x
+        // 60 and ten of 70 x 70, 8 iterations: 0.73 ms, one after the other
+        // 1.15, all with 4 waves in one launch 0.96; 128 of 64 x 64 and 128 of
+        // 65 x 65: 1.10, 1.58, 1.17)
+        const bool both = ns > 0 && ns < n;
+        if (both) {
+            st = hipEventRecord(e.ev_fork, e.stream);
+            if (st == hipSuccess) st = hipStreamWaitEvent(e.side, e.ev_fork, 0);
+            if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run fork");
+        }
+        if constexpr (BatchCGWaves<R>::MOST > 4)
+            if (ns < n)
+                rc = batch_cg_launch<R, LL, BatchCGWaves<R>::MOST>(e, e.stream, d_inst + ns, d_state + CG_NSTATE * ns,
+                                                                  n - ns, iters, max_iters, rtol, stall_iters);
+        if (!rc && ns > 0)
+            rc = batch_cg_launch<R, LL, 4>(e, both ? e.side : e.stream, d_inst, d_state, ns, iters, max_iters, rtol,
+                                           stall_iters);
         if (rc) return rc;
+        if (both) {
+            st = hipEventRecord(e.ev_join, e.side);
+            if (st == hipSuccess) st = hipStreamWaitEvent(e.stream, e.ev_join, 0);
+            if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run join");
+        }
         st = hipMemcpyAsync(hs.data(), d_state, sizeof(double) * CG_NSTATE * n, hipMemcpyDeviceToHost, e.stream);
         if (st == hipSuccess) st = hipStreamSynchronize(e.stream);
         if (st != hipSuccess) return check_hip(st, "glx_batch_cg_run readback");
