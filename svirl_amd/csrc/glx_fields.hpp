@@ -795,28 +795,19 @@ __device__ __forceinline__ Cells cells_from(const Geo &g, bool has_mt, int i, in
     return c;
 }
 
-template <typename R, bool withA, bool UPD = false>
+template <typename R, bool withA>
 __device__ __forceinline__ void grad_node(const Geo &g, const GeoR<R> &q, R kappa2, R eps, const R *eps_map, R H,
                                           const uint8_t *mt, const cplx<R> *psi, const R *abei, const R *ab, long n,
                                           int i, int j, R &e, cplx<R> &gj, R &ga, R &gb, bool &has_a, bool &has_b,
-                                          R bscale = R(1), const StateUpdate<R> *S = nullptr) {
+                                          R bscale = R(1)) {
     GradIn<R> in;
     // loads
     const long row = (long)g.Nx * j;
-    auto lp = [&](long k) {
-        cplx<R> p = ld(psi, k);
-        if constexpr (UPD) {
-            const cplx<R> d = ld(S->dpsi, k);
-            p.re = S->ap * d.re + p.re;
-            p.im = S->ap * d.im + p.im;
-        }
-        return p;
-    };
-    in.p0 = lp(n);
-    in.pl = lp(row + max(i - 1, 0));
-    in.pr = lp(row + min(i + 1, g.Nx - 1));
-    in.pd = lp((long)g.Nx * max(j - 1, 0) + i);
-    in.pu = lp((long)g.Nx * min(j + 1, g.Ny - 1) + i);
+    in.p0 = ld(psi, n);
+    in.pl = ld(psi, row + max(i - 1, 0));
+    in.pr = ld(psi, row + min(i + 1, g.Nx - 1));
+    in.pd = ld(psi, (long)g.Nx * max(j - 1, 0) + i);
+    in.pu = ld(psi, (long)g.Nx * min(j + 1, g.Ny - 1) + i);
     in.ee = eps_map ? eps_map[n] : eps;
     bool m_mm = true, m_mp = true, m_pm = true, m_pp = true;
     if (mt) {
@@ -834,25 +825,6 @@ __device__ __forceinline__ void grad_node(const Geo &g, const GeoR<R> &q, R kapp
     B = Links10<R>{};
     if (he) E = load_links10(g, abei, i, j);
     if (hb) B = load_links10(g, ab, i, j);
-    if constexpr (UPD) {
-        st(S->psi_out, n, in.p0);
-        if (S->dab) {
-            const Links10<R> d = load_links10(g, S->dab, i, j);
-            const R a = S->aa;
-            B.a00 = a * d.a00 + B.a00;
-            B.am0 = a * d.am0 + B.am0;
-            B.a0m = a * d.a0m + B.a0m;
-            B.a0p = a * d.a0p + B.a0p;
-            B.amp = a * d.amp + B.amp;
-            B.b00 = a * d.b00 + B.b00;
-            B.b0m = a * d.b0m + B.b0m;
-            B.bm0 = a * d.bm0 + B.bm0;
-            B.bp0 = a * d.bp0 + B.bp0;
-            B.bpm = a * d.bpm + B.bpm;
-            if (i < g.Nxa) S->ab_out[i + (long)g.Nxa * j] = B.a00;
-            if (j < g.Nyb) S->ab_out[g.Na + i + (long)g.Nxb * j] = B.b00;
-        }
-    }
     auto pvv = [&](R ve, R vb) {  // pv(abei, ab, k) of loaded values
         R p = R(0);
         if (he) p += ve;
@@ -866,60 +838,6 @@ __device__ __forceinline__ void grad_node(const Geo &g, const GeoR<R> &q, R kapp
     if (c.mm || c.mp) sincos_r(-q.dx * pvv(E.am0, B.am0), &in.sl, &in.cl);
     if (c.mm || c.pm) sincos_r(-q.dy * pvv(E.b0m, B.b0m), &in.sd, &in.cd);
     grad_eval<R, withA>(g, q, kappa2, H, he, hb, in, i, j, e, gj, ga, gb, has_a, has_b, bscale);
-}
-
-// One pass of the CG loop over the state (phase 1 of an iteration): writes
-// both Jacobians (overwriting, equal to the reference's += into a zeroed
-// buffer), and accumulates the free energy of the state and the two pairs
-// of Polak-Ribiere sums against the previous Jacobians. partials per
-// workgroup: F, num_psi, den_psi, num_A, den_A. withA: kappa < inf.
-template <typename R, bool withA, bool UPD = false>
-__global__ void __launch_bounds__(256) k_cg_gradient_pass(Geo g, R kappa2, R eps, const R *eps_map, R H, const uint8_t *mt,
-                                   const cplx<R> *psi, const R *abei, const R *ab, cplx<R> *jac,
-                                   const cplx<R> *jac_prev, R *jacA, const R *jacA_prev, double *partials,
-                                   StateUpdate<R> S = {}, const double *alpha = nullptr) {
-    const GeoR<R> q(g);
-    if constexpr (UPD) {
-        S.ap = R(alpha[0]);
-        S.aa = R(alpha[1]);
-    }
-    const R dxdy = q.dx * q.dy, s2 = R(2) * q.dx * q.dy;
-    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (long n = blockIdx.x * (long)blockDim.x + threadIdx.x; n < g.N; n += (long)gridDim.x * blockDim.x) {
-        int i, j;
-        node_ij(g, n, i, j);
-        R e, ga, gb;
-        cplx<R> gj;
-        bool ha, hb;
-        grad_node<R, withA, UPD>(g, q, kappa2, eps, eps_map, H, mt, psi, abei, ab, n, i, j, e, gj, ga, gb, ha, hb,
-                                 R(1), &S);
-        // every load of the node before its stores
-        const cplx<R> gp = ld(jac_prev, n);
-        const long la = i + (long)g.Nxa * j, lb = g.Na + i + (long)g.Nxb * j;
-        const R vpa = (withA && ha) ? jacA_prev[la] : R(0), vpb = (withA && hb) ? jacA_prev[lb] : R(0);
-        acc[0] += double(e);
-        const cplx<R> gv = {dxdy * gj.re, dxdy * gj.im};
-        st(jac, n, gv);
-        acc[1] += double(gv.re * (gv.re - gp.re));
-        acc[1] += double(gv.im * (gv.im - gp.im));
-        acc[2] += double(gp.re * gp.re);
-        acc[2] += double(gp.im * gp.im);
-        if (withA) {
-            if (ha) {
-                const R v = s2 * ga;
-                jacA[la] = v;
-                acc[3] += double(v * (v - vpa));
-                acc[4] += double(vpa * vpa);
-            }
-            if (hb) {
-                const R v = s2 * gb;
-                jacA[lb] = v;
-                acc[3] += double(v * (v - vpb));
-                acc[4] += double(vpb * vpb);
-            }
-        }
-    }
-    block_store_partials<5>(acc, partials);
 }
 
 // Where a gradient pass leaves its sums: the free energy (the first sum

@@ -94,10 +94,12 @@ class TD:
         return garray.device_pool()
 
     def _default_wg(self):
-        """Persistent grid: fewer workgroups for small grids (about 32 rows
-        per wave); 0 (the library's default: two workgroups per CU for the
-        psi solve and three for the A solve, the measured optima at 4097^2)
-        once a grid fills two workgroups per CU."""
+        """The workgroups that glx_td_run gives its row-marching solves: fewer
+        for small grids (about 32 rows per wave); 0 (two workgroups per CU for
+        the psi solve and three for the A solve, the measured optima at
+        4097^2) once a grid fills two workgroups per CU. A caller sets
+        self.wg to it to have a grid that fits the register tiles swept by
+        rows."""
         cfg = self.cfg
         strips = -(-int(cfg.Nx) // 62)
         rows = strips * int(cfg.Ny)
