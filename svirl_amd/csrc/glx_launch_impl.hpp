@@ -475,11 +475,16 @@ static int td_run_tiles(const Env &e, const TilePlan &pl, glx_grid g, const glx_
 // The tile shapes (rows per wave, halo, waves) of a precision. Few rows and
 // a narrow halo where the grid is small: more workgroups, each sweep short.
 // Many rows and waves where it is large: less of a tile is halo, and more
-// grids fit. The registers end the list: FP32 takes nine a node and spills
-// from 18 rows on, FP64 fourteen (and 24 bytes of LDS), from 9 on in the psi
-// sweeps. Measured per step (about 22 psi and 4 A sweeps; kappa = 5), row-marching
-// solves against tiles: FP32 129^2 276 / 43 us, 513^2 305 / 57, 1025^2 319 /
-// 94; FP64 129^2 444 / 48, 513^2 470 / 80, 771 x 1283 506 / 174.
+// grids fit. The registers end the list: FP32 takes nine a node (and 8 bytes
+// of LDS), all 256 with none spilled at 16 rows; FP64 fourteen (and 24 bytes
+// of LDS, 157 of 160 KB at 10 rows): with A, 8 rows spill 46 and 10 rows 111,
+// moved once a solve or step but for four accesses in the 10 rows' loop of psi
+// sweeps. That shape is there to hold the most nodes, so its halo is 4: 56 x
+// 72 nodes of its own, with a halo of 6 52 x 68; 771 x 1283 takes 252 of them,
+// 1024^2 and 1025^2 285, where 256 fit. Measured per step (about 22 psi and 4 A
+// sweeps; kappa = 5), row-marching solves against tiles: FP32 129^2 276 / 42
+// us, 513^2 305 / 56, 1025^2 319 / 91; FP64 129^2 444 / 47, 513^2 470 / 81,
+// 771 x 1283 506 / 173.
 template <typename R> struct TileShapes { using list = std::tuple<TileOf<4, 4, 4>, TileOf<8, 6, 4>, TileOf<12, 8, 4>, TileOf<14, 8, 8>, TileOf<16, 8, 8>>; };
 template <> struct TileShapes<double> { using list = std::tuple<TileOf<4, 4, 4>, TileOf<5, 5, 8>, TileOf<8, 6, 8>, TileOf<10, 4, 8>>; };
 
