@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 from scipy.ndimage import gaussian_filter
 
-from tests.test_gpu_tiles import run
+from tests.test_gpu_tiles import run, state
 
 pytestmark = pytest.mark.gpu
 nat = pytest.importorskip("svirl_amd._native")
@@ -41,3 +41,21 @@ def test_fp32_error_is_that_of_rows(size, kappa):
         assert wg or np.array_equal(sw[:, 0], sw64[:, 0])
         err.append(np.linalg.norm(p - ref) / np.linalg.norm(ref))
     assert err[0] <= 1.1 * err[1]
+
+
+# solves that end before, at and after the turn (the sweep limit), and steps of
+# few sweeps, which carry changes from the first one on
+@pytest.mark.parametrize("dt,max_sweeps", [(0.1, 1), (0.1, 2), (0.1, 3), (0.1, 4), (0.1, 9), (1e-3, 1024), (4e-3, 1024),
+                                           (1e-2, 1024)])
+@pytest.mark.parametrize("kappa", [0.0, 5.0])
+def test_fp32_short_solves(dt, max_sweeps, kappa):
+    """Six steps stay within 5e-7 of 64 bits: each is rounded some ten times
+    at 3e-8 of psi, in sums that the next steps do not amplify."""
+    Nx, Ny = 150, 131
+    f = state(Nx, Ny, np.float32, True, seed=9)
+    f64 = (f[0].astype(complex), f[1].astype(float), f[2], f[3].astype(float))
+    ref, ab64, sw64 = run(Nx, Ny, np.float64, f64, kappa, 8, 6, dt=dt, max_sweeps=max_sweeps)
+    p, ab, sw = run(Nx, Ny, np.float32, f, kappa, 0, 6, dt=dt, max_sweeps=max_sweeps)
+    assert np.array_equal(sw[:, 0], sw64[:, 0])
+    assert np.linalg.norm(p - ref) <= 5e-7 * np.linalg.norm(ref)
+    assert np.linalg.norm(ab - ab64) <= 5e-7 * np.linalg.norm(ab64)
